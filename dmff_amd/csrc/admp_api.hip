@@ -19,6 +19,7 @@
 #include "pair_kernels.h"
 #include "recip_kernels.h"
 #include "recip2_kernels.h"
+#include "recip_mm_kernels.h"
 #include "site_kernels.h"
 
 using namespace admp;
@@ -33,6 +34,8 @@ struct Grid {
     void* tw64[3] = {nullptr, nullptr, nullptr}; // double twiddles (used by the FP64 grids)
     double* bmod[3] = {nullptr, nullptr, nullptr};
     bool plane[2] = {false, false};  // fused plane FFT pass usable ([0] float, [1] double arithmetic)
+    bool mm = false;                 // FP64 passes on the matrix cores (recip_mm_kernels.h)
+    bool mm_plane = false;           // with the (x, y) plane in LDS
 };
 
 }  // namespace
@@ -99,7 +102,11 @@ struct admp_ctx {
     long blist_cap = 0;
     int* d_scan_tmp = nullptr;  // tile totals of scan_rows
     size_t scan_cap = 0;
+    int *d_tcount = nullptr, *d_tstart = nullptr;  // the same per (column tile, z segment) of k_spread_z
+    int2* d_tlist = nullptr;
+    long tlist_cap = 0;
     const Grid* prepped = nullptr;  // grid whose site bases / sort are current
+    bool bricks_ok = false, tiles_ok = false;   // and whose candidate lists are
     double* d_part = nullptr;   // influence partials
     int part_blocks = 0;
     double* d_rec = nullptr;    // F x 7 reduced influence sums
@@ -127,6 +134,7 @@ struct admp_ctx {
     int dots_blocks = 64;
     double* d_pparts = nullptr;               // CG partials (CgParts layout)
     int cg_nw = 0;                            // z.w slots per frame
+    int gz_tiles = 0;                         // column tiles of the largest matrix-core grid
     int cg_nwu = 0;                           // z.w slots written by the last product
     double *d_swfrac = nullptr, *d_sfq = nullptr;  // solver spline coordinates / fractional dipoles (R-typed)
     int pcg_nb = 0;
@@ -392,6 +400,64 @@ static bool plane_kernels_ready() {
     return ok;
 }
 
+// The same for the matrix-core passes, whose workgroups may take most of a CU's LDS.
+constexpr size_t MM_LDS_MAX = 156 * 1024;
+static bool mm_kernels_ready() {
+    static const bool ok = [] {
+        int dev = 0, lim = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&lim, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess ||
+            (size_t)lim < MM_LDS_MAX + 1024) {
+            (void)hipGetLastError();
+            return false;
+        }
+        const void* k[] = {(const void*)k_spread_z<0, false>, (const void*)k_spread_z<1, false>,
+                           (const void*)k_spread_z<2, false>, (const void*)k_spread_z<0, true>,
+                           (const void*)k_spread_z<1, true>, (const void*)k_spread_z<2, true>,
+                           (const void*)k_gather_z<0>, (const void*)k_gather_z<1>, (const void*)k_gather_z<2>,
+#define ADMP_MM_NT(NTv)                                                                                               \
+    (const void*)k_plane_mm<NTv, IN_TABLE>, (const void*)k_plane_mm<NTv, IN_TABLE_ACC>,                              \
+        (const void*)k_plane_mm<NTv, IN_ACC>, (const void*)k_plane_mm_matvec<NTv>, (const void*)k_y_mm<NTv>,          \
+        (const void*)k_x_mm<NTv, IN_TABLE>, (const void*)k_x_mm<NTv, IN_TABLE_ACC>, (const void*)k_x_mm<NTv, IN_ACC>
+                           ADMP_MM_NT(1), ADMP_MM_NT(2), ADMP_MM_NT(3), ADMP_MM_NT(4), ADMP_MM_NT(5)};
+#undef ADMP_MM_NT
+        static_assert(MM_NT == 5, "one instance per number of row tiles");
+        for (const void* f : k)
+            if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)MM_LDS_MAX) != hipSuccess) {
+                (void)hipGetLastError();
+                return false;
+            }
+        return true;
+    }();
+    return ok;
+}
+
+// ADMP_SPREAD=list|col|cw forces a spread of the radix path (measurements)
+static int spread_forced() {
+    static const int v = [] {
+        const char* e = std::getenv("ADMP_SPREAD");
+        if (!e) return 0;
+        if (std::strcmp(e, "list") == 0) return 1;
+        if (std::strcmp(e, "col") == 0) return 2;
+        if (std::strcmp(e, "cw") == 0) return 3;
+        return 0;
+    }();
+    return v;
+}
+
+// wavefronts sharing a z segment's candidates in k_spread_z
+static int spread_wpt(int K0, int K1, int K2, int F, int lm) {
+    const int nseg = mm_nseg(K2);
+    const long tiles = (long)((K0 + MM_TX - 1) / MM_TX) * ((K1 + MM_TY - 1) / MM_TY) * F;
+    
+    auto lds = [&](int n) {
+        return lm == 0 ? spread_mm_lds<0>(K2, n) : lm == 1 ? spread_mm_lds<1>(K2, n) : spread_mm_lds<2>(K2, n);
+    };
+    int w = 1;
+    while (w < 4 && 2 * w * nseg <= 16 && tiles * nseg * w < 2048 && lds(2 * w) <= MM_LDS_MAX) w *= 2;
+    return w;
+}
+
 static admp_status setup_grid(admp_ctx* ctx, Grid& g, int K0, int K1, int K2, bool mixed) {
     g.K[0] = K0; g.K[1] = K1; g.K[2] = K2;
     g.G = (size_t)K0 * K1 * K2;
@@ -432,6 +498,11 @@ static admp_status setup_grid(admp_ctx* ctx, Grid& g, int K0, int K1, int K2, bo
     // tables in LDS.  It is used up to PLANE_LDS_MAX bytes (two blocks per CU;
     // up to 50^2 in FP64, 71^2 in FP32); larger planes take the line passes.
     const char* env = std::getenv("ADMP_FFT_PLANE");
+    // The FP64 passes run on the matrix cores up to MM_KMAX points per axis, with the
+    // plane in LDS where it fits one workgroup per CU.
+    g.mm = K0 <= MM_KMAX && K1 <= MM_KMAX && K2 <= MM_KMAX && K0 >= BRX + 5 && K1 >= BRY + 5 && K2 >= BRZ + 5 &&
+           !spread_forced() && mm_kernels_ready();
+    g.mm_plane = g.mm && plane_mm_lds(K0, K1) <= MM_PLANE_LDS && !(env && env[0] == '0');
     const bool allow = !(env && env[0] == '0') && K0 >= BRX + 5 && K1 >= BRY + 5 && K2 >= BRZ + 5;
     for (int w = 0; w < 2; ++w) {
         const size_t cs = w ? sizeof(Cplx<double>) : sizeof(Cplx<float>);
@@ -636,7 +707,7 @@ extern "C" admp_status admp_ctx_create(const admp_config* cfg, admp_ctx** out) {
         for (const Grid* gg : {&ctx->eg, &ctx->dg})
             if (gg->G) {
                 Hmax = std::max(Hmax, (size_t)gg->K[0] * gg->K[1] * (gg->K[2] / 2 + 1));
-                Lmax = std::max(Lmax, (size_t)gg->K[1] * (gg->K[2] / 2 + 1));
+                Lmax = std::max(Lmax, (size_t)gg->K[1] * (gg->K[2] / 2 + 1));  // blocks of any x pass
             }
         ALLOC(g, Hmax * 2 * ctx->F);
         ctx->d_hgrid = g;
@@ -646,17 +717,32 @@ extern "C" admp_status admp_ctx_create(const admp_config* cfg, admp_ctx** out) {
         ALLOC(ctx->d_gccount, Gmax * ctx->F);
         ALLOC(ctx->d_gcfill, Gmax * ctx->F);
         ALLOC(ctx->d_gcstart, (Gmax + 1) * ctx->F);
-        size_t nbrmax = 0;
+        // brick lists for the radix path (FP32 passes, grids beyond the matrix-core
+        // passes), tile lists for the matrix-core passes
+        size_t nbrmax = 0, ntmax = 0;
         for (const Grid* gg : {&ctx->eg, &ctx->dg})
-            if (gg->G)
-                nbrmax = std::max(nbrmax, (size_t)((gg->K[0] + BRX - 1) / BRX) * ((gg->K[1] + BRY - 1) / BRY) *
-                                              ((gg->K[2] + BRZ - 1) / BRZ));
-        ALLOC(ctx->d_bcount, nbrmax * ctx->F);
-        ALLOC(ctx->d_bstart, (nbrmax + 1) * ctx->F);
+            if (gg->G) {
+                const size_t nxy = (size_t)((gg->K[0] + BRX - 1) / BRX) * ((gg->K[1] + BRY - 1) / BRY);
+                if (mixed || !gg->mm) nbrmax = std::max(nbrmax, nxy * ((gg->K[2] + BRZ - 1) / BRZ));
+                if (gg->mm) {
+                    ntmax = std::max(ntmax, nxy * mm_nseg(gg->K[2]));
+                    ctx->gz_tiles = std::max(ctx->gz_tiles, (int)nxy);
+                }
+            }
+        if (nbrmax) {
+            ALLOC(ctx->d_bcount, nbrmax * ctx->F);
+            ALLOC(ctx->d_bstart, (nbrmax + 1) * ctx->F);
+            ctx->blist_cap = (long)BRICK_MAXCAND * ctx->N;  // per frame
+            ALLOC(ctx->d_blist, (size_t)ctx->blist_cap * ctx->F);
+        }
+        if (ntmax) {
+            ALLOC(ctx->d_tcount, ntmax * ctx->F);
+            ALLOC(ctx->d_tstart, (ntmax + 1) * ctx->F);
+            ctx->tlist_cap = (long)MM_TILE_COPIES * ctx->N;  // per frame
+            ALLOC(ctx->d_tlist, (size_t)ctx->tlist_cap * ctx->F);
+        }
         if (ctx->eg.G)
             ALLOC(ctx->d_infl, (size_t)ctx->eg.K[0] * ctx->eg.K[1] * (ctx->eg.K[2] / 2 + 1) * ctx->F);
-        ctx->blist_cap = (long)BRICK_MAXCAND * ctx->N;  // per frame
-        ALLOC(ctx->d_blist, (size_t)ctx->blist_cap * ctx->F);
     }
     ALLOC(ctx->d_wd, NF * 3);
     ALLOC(ctx->d_gcell, NF);
@@ -672,7 +758,7 @@ extern "C" admp_status admp_ctx_create(const admp_config* cfg, admp_ctx** out) {
     ALLOC(ctx->d_dpart, (size_t)ctx->dots_blocks * ctx->F * 3);
     ALLOC(ctx->d_dots, ctx->F * 3);
     ctx->pcg_nb = (int)nblk(ctx->N, PCG_BLOCK);
-    ctx->cg_nw = std::max(ctx->pcg_nb, gather_blocks(ctx->N));
+    ctx->cg_nw = std::max({ctx->pcg_nb, gather_blocks(ctx->N), ctx->gz_tiles});
     ALLOC(ctx->d_pparts, (size_t)ctx->F * (ctx->cg_nw + 4 * ctx->pcg_nb));
     ALLOC(ctx->d_s, NF * 6);
     ALLOC(ctx->d_pnear, NF); ALLOC(ctx->d_pcj, NF * 3); ALLOC(ctx->d_pcd, NF * 3 * PC_ROW);
@@ -836,7 +922,8 @@ static admp_status ensure_cap(admp_ctx* ctx, int need) {
 // ADMP_ERR_ARG from geom_check() after it.
 static admp_status upload_geometry(admp_ctx* ctx, const double* pos, const double* box) {
     const size_t NF = (size_t)ctx->N * ctx->F;
-    ctx->prepped = nullptr;  // site grid bases / sort follow the positions
+    ctx->prepped = nullptr;  // site grid bases, sort and lists follow the positions
+    ctx->bricks_ok = ctx->tiles_ok = false;
     HIPCHK(hipMemsetAsync(ctx->d_geom, 0, sizeof(int), ctx->stream));
     hipLaunchKernelGGL(k_pack_pos, dim3(nblk(NF, 256)), dim3(256), 0, ctx->stream, NF, pos, ctx->d_pos, ctx->d_geom);
     const admp_config& c = ctx->cfg;
@@ -1141,20 +1228,10 @@ static admp_status recip_positions(admp_ctx* ctx, const Grid& g, int use_dA) {
                            ctx->d_gcstart, ctx->d_gcfill, ctx->d_gcatoms, 0);
         hipLaunchKernelGGL(k_cell_sort, dim3(nblk(G, 256), F), dim3(256), 0, st, (int)G, N, ctx->d_gcstart,
                            ctx->d_gcatoms);
-        // per-brick candidate lists for the spreads of this evaluation
-        const int nbr = ((g.K[0] + BRX - 1) / BRX) * ((g.K[1] + BRY - 1) / BRY) * ((g.K[2] + BRZ - 1) / BRZ);
-        hipLaunchKernelGGL(k_brick_cands<false>, dim3(nbr, F), dim3(64), 0, st, N, g.K[0], g.K[1], g.K[2],
-                           ctx->d_mbase, ctx->d_gcstart, ctx->d_gcatoms, ctx->d_bcount, (const int*)nullptr,
-                           (int2*)nullptr, 0L);
-        s2 = scan_rows(ctx, ctx->d_bcount, ctx->d_bstart, nbr, F, st);
-        if (s2 != ADMP_OK) return s2;
-        hipLaunchKernelGGL(k_brick_cands<true>, dim3(nbr, F), dim3(64), 0, st, N, g.K[0], g.K[1], g.K[2],
-                           ctx->d_mbase, ctx->d_gcstart, ctx->d_gcatoms, ctx->d_bcount, ctx->d_bstart, ctx->d_blist,
-                           ctx->blist_cap);
         if (&g == &ctx->eg && ctx->d_infl && !use_dA) {
             const size_t nt = (size_t)g.K[0] * g.K[1] * (g.K[2] / 2 + 1);
             // laid out for the FP64 solver products' FFT path
-            ctx->infl_pm = g.plane[1] ? 1 : 0;
+            ctx->infl_pm = g.mm || g.plane[1] ? 1 : 0;
             hipLaunchKernelGGL(k_infl_table, dim3(nblk(nt, 256), F), dim3(256), 0, st, g.K[0], g.K[1], g.K[2],
                                ctx->d_box, g.bmod[0], g.bmod[1], g.bmod[2], ctx->cfg.kappa, DIELECTRIC, ctx->infl_pm,
                                ctx->d_infl);
@@ -1163,8 +1240,34 @@ static admp_status recip_positions(admp_ctx* ctx, const Grid& g, int use_dA) {
     }
     HIPCHK(hipGetLastError());
     ctx->prepped = &g;
+    ctx->bricks_ok = ctx->tiles_ok = false;
     return ADMP_OK;
 }
+
+// candidate lists of the radix path's bricks, or of the matrix-core passes' tiles
+static admp_status recip_lists(admp_ctx* ctx, const Grid& g, bool tiles) {
+    bool& ok = tiles ? ctx->tiles_ok : ctx->bricks_ok;
+    if (ok) return ADMP_OK;
+    const int N = ctx->N, F = ctx->F;
+    hipStream_t st = ctx->stream;
+    ProfScope ps_(ctx, 3);
+    const int lz = tiles ? mm_seglen(g.K[2]) : BRZ;
+    const int nbr = ((g.K[0] + BRX - 1) / BRX) * ((g.K[1] + BRY - 1) / BRY) * ((g.K[2] + lz - 1) / lz);
+    int* count = tiles ? ctx->d_tcount : ctx->d_bcount;
+    int* start = tiles ? ctx->d_tstart : ctx->d_bstart;
+    int2* list = tiles ? ctx->d_tlist : ctx->d_blist;
+    const long cap = tiles ? ctx->tlist_cap : ctx->blist_cap;
+    hipLaunchKernelGGL(k_brick_cands<false>, dim3(nbr, F), dim3(64), 0, st, N, g.K[0], g.K[1], g.K[2], lz, (int)tiles,
+                       ctx->d_mbase, ctx->d_gcstart, ctx->d_gcatoms, count, (const int*)nullptr, (int2*)nullptr, 0L);
+    const admp_status s = scan_rows(ctx, count, start, nbr, F, st);
+    if (s != ADMP_OK) return s;
+    hipLaunchKernelGGL(k_brick_cands<true>, dim3(nbr, F), dim3(64), 0, st, N, g.K[0], g.K[1], g.K[2], lz, (int)tiles,
+                       ctx->d_mbase, ctx->d_gcstart, ctx->d_gcatoms, count, start, list, cap);
+    HIPCHK(hipGetLastError());
+    ok = true;
+    return ADMP_OK;
+}
+
 
 template <class R> static const Cplx<R>* twid(const Grid& g, int d) {
     return reinterpret_cast<const Cplx<R>*>(sizeof(R) == 8 ? g.tw64[d] : g.tw[d]);
@@ -1176,6 +1279,137 @@ struct MatvecJob {
     const double* v;
     double* out;
 };
+
+// The FP64 spread, transforms and gather on the matrix cores (recip_mm_kernels.h);
+// arguments as recip_run's, with the spline coordinates and fractional multipoles
+// already formed.
+static admp_status recip_run_mm(admp_ctx* ctx, const Grid& g, int use_dA, const double* Qc, const double* U, int qmode,
+                                int lmax_eff, int kind, double pref, double kappa, int gather_mode, double* out3,
+                                double* gq, double* gpos, double* vir, bool want_energy, const double* wfrac,
+                                const double* fq, const PcgState* skip, const CgEpi* epi, hipEvent_t before_gather,
+                                const MatvecJob* mv) {
+    const int N = ctx->N, F = ctx->F;
+    hipStream_t st = ctx->stream;
+    admp_status s = recip_lists(ctx, g, true);
+    if (s != ADMP_OK) return s;
+    const int K0 = g.K[0], K1 = g.K[1], K2 = g.K[2], H = K2 / 2 + 1;
+    Cplx<double>* hg = reinterpret_cast<Cplx<double>*>(ctx->d_hgrid);
+    const unsigned tiles = xcd_blocks(((K0 + MM_TX - 1) / MM_TX) * ((K1 + MM_TY - 1) / MM_TY));
+    {
+        ProfScope ps_(ctx, 4);
+        const int lm = std::min(lmax_eff, 2), wpt = spread_wpt(K0, K1, K2, F, lm);
+        const dim3 grid(tiles, F), block(64 * mm_nseg(K2) * wpt);
+#define ADMP_SPREAD_Z(LMv)                                                                                            \
+    if (mm_nseg(K2) == 1)                                                                                            \
+        hipLaunchKernelGGL((k_spread_z<LMv, true>), grid, block, spread_mm_lds<LMv>(K2, wpt), st, N, K0, K1, K2, wpt, \
+                           twid<double>(g, 2), wfrac, fq, ctx->d_tstart, ctx->d_tlist, ctx->tlist_cap, hg, skip,     \
+                           ctx->spread_chk);                                                                         \
+    else                                                                                                             \
+        hipLaunchKernelGGL((k_spread_z<LMv, false>), grid, block, spread_mm_lds<LMv>(K2, wpt), st, N, K0, K1, K2,     \
+                           wpt, twid<double>(g, 2), wfrac, fq, ctx->d_tstart, ctx->d_tlist, ctx->tlist_cap, hg, skip, \
+                           ctx->spread_chk);
+        if (lm == 2) { ADMP_SPREAD_Z(2) }
+        else if (lm == 1) { ADMP_SPREAD_Z(1) }
+        else { ADMP_SPREAD_Z(0) }
+#undef ADMP_SPREAD_Z
+    }
+    const bool use_tab = &g == &ctx->eg && kind == 0 && !use_dA && pref == DIELECTRIC && kappa == ctx->cfg.kappa &&
+                         ctx->d_infl && ctx->infl_pm;
+    const InflArgs q{ctx->d_box, g.bmod[0], g.bmod[1], g.bmod[2], kappa, kind, pref, ctx->d_infl, ctx->d_part};
+    // without the table (another grid or kind than the solver's) the function is computed
+    const int in = !use_tab ? IN_ACC : want_energy ? IN_TABLE_ACC : IN_TABLE;
+    const int ntx = mm_tiles(K0), nty = mm_tiles(K1);
+    int npart = H;
+    // f(row tiles) with the row tiles as a constant
+    auto with_nt = [](int n, auto f) {
+        switch (n) {
+            case 1: f(std::integral_constant<int, 1>()); break;
+            case 2: f(std::integral_constant<int, 2>()); break;
+            case 3: f(std::integral_constant<int, 3>()); break;
+            case 4: f(std::integral_constant<int, 4>()); break;
+            default: f(std::integral_constant<int, 5>()); break;
+        }
+    };
+    if (g.mm_plane) {
+        ProfScope ps_(ctx, mv ? 13 : 6);
+        const size_t sm = plane_mm_lds(K0, K1);
+        const int th = plane_mm_threads(K0, K1);
+        const Cplx<double>*tx = twid<double>(g, 0), *ty = twid<double>(g, 1);
+        with_nt(std::max(ntx, nty), [&](auto n) {
+            constexpr int NT = decltype(n)::value;
+            if (mv) {
+                const int npb = xcd_blocks(H * F), nbf = (int)nblk((size_t)N * TPA, th);
+                hipLaunchKernelGGL(k_plane_mm_matvec<NT>, dim3(npb + xcd_blocks(nbf * F)), dim3(th), sm, st, K0, K1, K2, tx,
+                                   ty, hg, q, F, npb, N, nbf, ctx->cap, ctx->d_pos, ctx->d_nbr, ctx->d_ncnt,
+                                   reinterpret_cast<const double*>(ctx->d_pcoef), mv->v, mv->out, skip);
+            } else if (in == IN_TABLE) {
+                hipLaunchKernelGGL((k_plane_mm<NT, IN_TABLE>), dim3(H, F), dim3(th), sm, st, K0, K1, K2, tx, ty, hg, q, skip);
+            } else if (in == IN_TABLE_ACC) {
+                hipLaunchKernelGGL((k_plane_mm<NT, IN_TABLE_ACC>), dim3(H, F), dim3(th), sm, st, K0, K1, K2, tx, ty, hg, q,
+                                   skip);
+            } else {
+                hipLaunchKernelGGL((k_plane_mm<NT, IN_ACC>), dim3(H, F), dim3(th), sm, st, K0, K1, K2, tx, ty, hg, q, skip);
+            }
+        });
+    } else {
+        if (mv) { ctx->err = "real-space product with the plane pass needs the plane in LDS"; return ADMP_ERR_STATE; }
+        const unsigned yb = nblk((size_t)H * K0, MM_LINES), xb = H * nblk(K1, MM_LINES);
+        auto ylines = [&](int inverse) {
+            ProfScope ps_(ctx, 5);
+            with_nt(nty, [&](auto n) {
+                constexpr int NT = decltype(n)::value;
+                hipLaunchKernelGGL(k_y_mm<NT>, dim3(yb, F), dim3(MM_LINE_THREADS), line_mm_lds(K1), st, K0, K1, H,
+                                   twid<double>(g, 1), hg, inverse, skip);
+            });
+        };
+        ylines(0);
+        {
+            ProfScope ps_(ctx, 6);
+            npart = (int)xb;
+            with_nt(ntx, [&](auto n) {
+                constexpr int NT = decltype(n)::value;
+                const dim3 gr(xb, F), bl(MM_LINE_THREADS);
+                const size_t sm = xline_mm_lds(K0);
+                const Cplx<double>* tx = twid<double>(g, 0);
+                if (in == IN_TABLE)
+                    hipLaunchKernelGGL((k_x_mm<NT, IN_TABLE>), gr, bl, sm, st, K0, K1, K2, tx, hg, q, skip);
+                else if (in == IN_TABLE_ACC)
+                    hipLaunchKernelGGL((k_x_mm<NT, IN_TABLE_ACC>), gr, bl, sm, st, K0, K1, K2, tx, hg, q, skip);
+                else
+                    hipLaunchKernelGGL((k_x_mm<NT, IN_ACC>), gr, bl, sm, st, K0, K1, K2, tx, hg, q, skip);
+            });
+        }
+        ylines(1);
+    }
+    if (want_energy)
+        hipLaunchKernelGGL(k_reduce_cols, dim3(7, F), dim3(RED_BLOCK), 0, st, npart, 7, ctx->d_part, ctx->d_rec, 0);
+    if (before_gather) HIPCHK(hipStreamWaitEvent(st, before_gather, 0));
+    {
+        ProfScope ps_(ctx, 7);
+        const CgEpi none{};
+        const int gt = gather_z_threads(tiles * F);
+        if (gather_mode == 2)
+            hipLaunchKernelGGL(k_gather_z<2>, dim3(tiles, F), dim3(gt), gather_z_lds<2>(K2, gt), st, N, K0, K1, K2, twid<double>(g, 2), ctx->d_pos,
+                               ctx->d_box, use_dA, ctx->d_mbase, wfrac, fq, Qc, U, qmode, hg, out3, gq, gpos, vir,
+                               ctx->d_gcstart, ctx->d_gcatoms, skip, *epi);
+        else if (gather_mode == 1)
+            hipLaunchKernelGGL(k_gather_z<1>, dim3(tiles, F), dim3(gt), gather_z_lds<1>(K2, gt), st, N, K0, K1, K2, twid<double>(g, 2), ctx->d_pos,
+                               ctx->d_box, use_dA, ctx->d_mbase, wfrac, fq, Qc, U, qmode, hg, out3, gq, gpos, vir,
+                               ctx->d_gcstart, ctx->d_gcatoms, skip, none);
+        else
+            hipLaunchKernelGGL(k_gather_z<0>, dim3(tiles, F), dim3(gt), gather_z_lds<0>(K2, gt), st, N, K0, K1, K2, twid<double>(g, 2), ctx->d_pos,
+                               ctx->d_box, use_dA, ctx->d_mbase, wfrac, fq, Qc, U, qmode, hg, out3, gq, gpos, vir,
+                               ctx->d_gcstart, ctx->d_gcatoms, skip, none);
+    }
+    HIPCHK(hipGetLastError());
+    return ADMP_OK;
+}
+
+// z.w partials the CG epilogue of the gather leaves per frame
+template <class R> static int gather_parts(const admp_ctx* ctx) {
+    const Grid& g = ctx->eg;
+    return sizeof(R) == 8 && g.mm ? ((g.K[0] + MM_TX - 1) / MM_TX) * ((g.K[1] + MM_TY - 1) / MM_TY) : gather_blocks(ctx->N);
+}
 
 // Spread the sources (Qc, U, qmode), transform, apply the influence function,
 // transform back and gather.  gather_mode 1: dE/dmu only into out3; 0: full
@@ -1198,6 +1432,11 @@ static admp_status recip_run(admp_ctx* ctx, const Grid& g, int use_dA, const dou
         ProfScope ps_(ctx, 3);
         hipLaunchKernelGGL(k_frac_mult<R>, dim3(nblk(N, 128), F), dim3(128), 0, st, N, ctx->d_box, use_dA, Qc, U, qmode,
                            ctx->d_wd, wfrac, fq);
+    }
+    if constexpr (sizeof(R) == 8) {
+        if (g.mm)
+            return recip_run_mm(ctx, g, use_dA, Qc, U, qmode, lmax_eff, kind, pref, kappa, gather_mode, out3, gq, gpos,
+                                vir, want_energy, wfrac, fq, skip, epi, before_gather, mv);
     }
     const int K0 = g.K[0], K1 = g.K[1], K2 = g.K[2];
     if (small_grid(g) && gather_mode == 2) {
@@ -1239,25 +1478,17 @@ static admp_status recip_run(admp_ctx* ctx, const Grid& g, int use_dA, const dou
         HIPCHK(hipGetLastError());
         return ADMP_OK;
     }
+    { const admp_status sl = recip_lists(ctx, g, false); if (sl != ADMP_OK) return sl; }
     R* rg = reinterpret_cast<R*>(ctx->d_rgrid);
     Cplx<R>* hg = reinterpret_cast<Cplx<R>*>(ctx->d_hgrid);
     const int H = K2 / 2 + 1;
     const int nbricks = ((K0 + BRX - 1) / BRX) * ((K1 + BRY - 1) / BRY) * ((K2 + BRZ - 1) / BRZ);
     { ProfScope ps_(ctx, 4);
-    // ADMP_SPREAD=list|col|cw forces one variant (measurements)
-    static const int spread_force = [] {
-        const char* e = std::getenv("ADMP_SPREAD");
-        if (!e) return 0;
-        if (std::strcmp(e, "list") == 0) return 1;
-        if (std::strcmp(e, "col") == 0) return 2;
-        if (std::strcmp(e, "cw") == 0) return 3;
-        return 0;
-    }();
     // default: one brick per wavefront with column accumulation (k_spread_cw); at
     // 12,288 sites it takes 19 us per solver spread where one grid point per lane
     // (list) takes 27 and four bricks per wavefront (col) 45, and it is also the
     // fastest for the 64-frame batch
-    const int variant = spread_force ? spread_force : 3;
+    const int variant = spread_forced() ? spread_forced() : 3;
     const unsigned nb1 = xcd_blocks(nbricks), nb4 = xcd_blocks((nbricks + 3) / 4);
 #define ADMP_SPREAD(LMv)                                                                                              \
     if (variant == 2)                                                                                                \
@@ -1446,7 +1677,8 @@ static admp_status pcg_apply(admp_ctx* ctx, const double* pol, double f1, int cu
     // real-space product then runs inside that launch (k_plane_matvec) instead of
     // on the side stream, which saves the fork and the join of every iteration.
     const int H = ctx->eg.K[2] / 2 + 1;
-    const bool with_plane = fused && sizeof(RC) == 8 && ctx->eg.plane[sizeof(R) == 8 ? 1 : 0] && H * F <= 128;
+    const bool plane = sizeof(R) == 8 && ctx->eg.mm ? ctx->eg.mm_plane : ctx->eg.plane[sizeof(R) == 8 ? 1 : 0];
+    const bool with_plane = fused && sizeof(RC) == 8 && plane && H * F <= 128;
     if (!with_plane) {
         // the real-space product runs on the side stream, beside the reciprocal chain
         HIPCHK(hipEventRecord(ctx->ev_fork, st));
@@ -1466,12 +1698,12 @@ static admp_status pcg_apply(admp_ctx* ctx, const double* pol, double f1, int cu
         const MatvecJob mv{ctx->d_z, ctx->d_t1};
         s = recip_run<R>(ctx, ctx->eg, 0, nullptr, ctx->d_z, 2, 1, 0, DIELECTRIC, ctx->cfg.kappa, 2, ctx->d_Ap,
                          nullptr, nullptr, nullptr, false, ctx->d_swfrac, ctx->d_sfq, ctx->d_pcg, &epi, nullptr, &mv);
-        ctx->cg_nwu = gather_blocks(N);
+        ctx->cg_nwu = gather_parts<R>(ctx);
     } else if (fused) {
         const CgEpi epi{ctx->d_t1, pol, f1, cg_parts(ctx)};
         s = recip_run<R>(ctx, ctx->eg, 0, nullptr, ctx->d_z, 2, 1, 0, DIELECTRIC, ctx->cfg.kappa, 2, ctx->d_Ap,
                          nullptr, nullptr, nullptr, false, ctx->d_swfrac, ctx->d_sfq, ctx->d_pcg, &epi, ctx->ev_join);
-        ctx->cg_nwu = gather_blocks(N);
+        ctx->cg_nwu = gather_parts<R>(ctx);
     } else if (ctx->cfg.lpme) {
         s = recip_run<R>(ctx, ctx->eg, 0, nullptr, ctx->d_z, 2, 1, 0, DIELECTRIC, ctx->cfg.kappa, 1, ctx->d_t2,
                          nullptr, nullptr, nullptr, false, ctx->d_swfrac, ctx->d_sfq, ctx->d_pcg);
@@ -1883,7 +2115,10 @@ static admp_status solve(admp_ctx* ctx, const double* pol, const double* thole, 
         if (s != ADMP_OK) return s;
         // a replayed set-up graph sorted the sites for the spread as well (the host
         // state its capture left): later launches and captures must not sort again
-        if (c.lpme) ctx->prepped = &ctx->eg;
+        if (c.lpme) {
+            ctx->prepped = &ctx->eg;
+            (ctx->eg.mm ? ctx->tiles_ok : ctx->bricks_ok) = true;
+        }
     } else {
         if ((s = launch_frames_fwd(ctx)) != ADMP_OK) return s;
         if ((s = solver_rhs<double, double>(ctx, pol, thole, pp)) != ADMP_OK) return s;

@@ -772,8 +772,8 @@ __device__ __forceinline__ void real_matvec_pairs(int sub, int cnt, const BoxInf
     for (int k = sub; k < cnt; k += TPA) term(nl[k] & NB_MASK, pc[2 * k], pc[2 * k + 1]);
 }
 
-template <class RC, class R, int BS>
-__device__ __forceinline__ void real_matvec_body(int item, int N, int nbf, int cap, const double4* __restrict__ pos,
+template <class RC, class R>
+__device__ __forceinline__ void real_matvec_body(int BS, int item, int N, int nbf, int cap, const double4* __restrict__ pos,
                                                  const BoxInfo* __restrict__ boxes, const int* __restrict__ nbr,
                                                  const int* __restrict__ ncnt, const RC* __restrict__ pcoef,
                                                  const R* __restrict__ v, double* __restrict__ out,
@@ -811,7 +811,7 @@ k_real_matvec(int N, int nbf, int F, int cap, const double4* __restrict__ pos, c
               const R* __restrict__ v, double* __restrict__ out, const PcgState* __restrict__ skip) {
     const int item = xcd_item(blockIdx.x, nbf * F);
     if (item >= nbf * F) return;
-    real_matvec_body<RC, R, PAIR_BLOCK>(item, N, nbf, cap, pos, boxes, nbr, ncnt, pcoef, v, out, skip);
+    real_matvec_body<RC, R>(PAIR_BLOCK, item, N, nbf, cap, pos, boxes, nbr, ncnt, pcoef, v, out, skip);
 }
 
 }  // namespace admp

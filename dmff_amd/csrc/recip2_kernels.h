@@ -105,26 +105,28 @@ constexpr int BRICK_MAXCAND = ((BRX + 5 + BRX - 1) / BRX + 1) * ((BRY + 5 + BRY 
 constexpr int BRICK_SEG = (BRX + 5) * (BRY + 5) * 2;   // column segments (two when z wraps)
 constexpr int BRICK_SEG_LANE = (BRICK_SEG + 63) / 64;   // segments per lane of the wavefront
 
+// lz: z points of a brick (BRZ, or the taller segments of k_spread_z); trim: a last
+// brick cut off by the grid lists only what can touch its points
 template <bool FILL>
 __global__ void __launch_bounds__(64)
-k_brick_cands(int N, int K0, int K1, int K2, const int4* __restrict__ mbase, const int* __restrict__ cstart,
-              const int* __restrict__ catoms, int* __restrict__ bcount, const int* __restrict__ bstart,
-              int2* __restrict__ blist, long cap) {
+k_brick_cands(int N, int K0, int K1, int K2, int lz, int trim, const int4* __restrict__ mbase,
+              const int* __restrict__ cstart, const int* __restrict__ catoms, int* __restrict__ bcount,
+              const int* __restrict__ bstart, int2* __restrict__ blist, long cap) {
     constexpr int NC = BRICK_SEG;
     constexpr int SL = BRICK_SEG_LANE;
     __shared__ int col_lo[NC];
     __shared__ int col_off[NC + 1];
     const int f = blockIdx.y;
-    const int nbz = (K2 + BRZ - 1) / BRZ, nby = (K1 + BRY - 1) / BRY, nbx = (K0 + BRX - 1) / BRX;
+    const int nbz = (K2 + lz - 1) / lz, nby = (K1 + BRY - 1) / BRY, nbx = (K0 + BRX - 1) / BRX;
     const int nbr = nbx * nby * nbz;
     const int b = blockIdx.x;
     const int bz = b % nbz, by = (b / nbz) % nby, bx = b / (nbz * nby);
-    const int X0 = bx * BRX, Y0 = by * BRY, Z0 = bz * BRZ;
+    const int X0 = bx * BRX, Y0 = by * BRY, Z0 = bz * lz;
     const int t = threadIdx.x;
     const size_t G = (size_t)K0 * K1 * K2;
     const int* cs = cstart + (size_t)f * (G + 1);
     const int* ca = catoms + (size_t)f * N;
-    const int nx = min(BRX + 5, K0), ny = min(BRY + 5, K1), nzr = min(BRZ + 5, K2);
+    const int nx = min(BRX + 5, K0), ny = min(BRY + 5, K1), nzr = min((trim ? min(lz, K2 - Z0) : lz) + 5, K2);
     const int nseg = nx * ny * 2;
     const int zs = wrapi(Z0 - 2, K2);
     const int zlen1 = min(nzr, K2 - zs), zlen2 = nzr - zlen1;
@@ -1103,6 +1105,124 @@ struct CgEpi {
 // eight lanes per site; 16 sites per block measured within ±1 % of 32, 8 slower
 constexpr int GATHER_SITES_PER_BLOCK = 32;
 
+// Outputs of one site from the derivatives fp[c][aa][bb] of its fractional potential
+// (orders below ND) in the gather's modes; zw: the site's z.w term is added (MODE 2)
+template <class R, int MODE>
+__device__ __forceinline__ void gather_site_out(size_t a, const double* A,
+                                                const double (&fp)[MODE == 0 ? 4 : 2][MODE == 0 ? 4 : 2][MODE == 0 ? 4 : 2],
+                                                const double4* __restrict__ pos, const R* __restrict__ fq,
+                                                const double* __restrict__ Qc, const double* __restrict__ U, int qmode,
+                                                double* __restrict__ out3, double* __restrict__ g_q,
+                                                double* __restrict__ g_pos, double* __restrict__ vir_atom, double e_pol,
+                                                const double* e_real, const double* e_z, double f1, double& zw) {
+    const double p1[3] = {fp[1][0][0], fp[0][1][0], fp[0][0][1]};
+    if constexpr (MODE == 2) {
+        const double ap = e_pol < 1e-8 ? 1e-8 : e_pol;
+        const double d = DIELECTRIC / ap - 2.0 * DIELECTRIC * f1;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const double dm = A[c * 3 + 0] * p1[0] + A[c * 3 + 1] * p1[1] + A[c * 3 + 2] * p1[2];
+            const double zv = e_z[c];
+            const double wv = e_real[c] + dm + d * zv;
+            out3[a * 3 + c] = wv;
+            zw += zv * wv;
+        }
+        return;
+    }
+    double dmu[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) dmu[c] = A[c * 3 + 0] * p1[0] + A[c * 3 + 1] * p1[1] + A[c * 3 + 2] * p1[2];
+    if constexpr (MODE == 1) {
+        out3[a * 3 + 0] = dmu[0]; out3[a * 3 + 1] = dmu[1]; out3[a * 3 + 2] = dmu[2];
+        return;
+    } else if constexpr (MODE == 0) {
+        double p2[3][3];
+        p2[0][0] = fp[2][0][0]; p2[1][1] = fp[0][2][0]; p2[2][2] = fp[0][0][2];
+        p2[0][1] = p2[1][0] = fp[1][1][0]; p2[0][2] = p2[2][0] = fp[1][0][1]; p2[1][2] = p2[2][1] = fp[0][1][1];
+        // third derivatives d3[j][k][l] (symmetric), from the ten independent entries
+        double d3[3][3][3];
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+#pragma unroll
+                for (int l = 0; l < 3; ++l) {
+                    const int ox = (j == 0) + (k == 0) + (l == 0);
+                    const int oy = (j == 1) + (k == 1) + (l == 1);
+                    const int oz = (j == 2) + (k == 2) + (l == 2);
+                    double v = 0;
+                    if (ox == 3) v = fp[3][0][0];
+                    else if (oy == 3) v = fp[0][3][0];
+                    else if (oz == 3) v = fp[0][0][3];
+                    else if (ox == 2 && oy == 1) v = fp[2][1][0];
+                    else if (ox == 2 && oz == 1) v = fp[2][0][1];
+                    else if (oy == 2 && ox == 1) v = fp[1][2][0];
+                    else if (oy == 2 && oz == 1) v = fp[0][2][1];
+                    else if (oz == 2 && ox == 1) v = fp[1][0][2];
+                    else if (oz == 2 && oy == 1) v = fp[0][1][2];
+                    else v = fp[1][1][1];
+                    d3[j][k][l] = v;
+                }
+        const R* c = fq + a * 10;
+        const double q = (double)c[0];
+        const double fm[3] = {(double)c[1], (double)c[2], (double)c[3]};
+        double fT[3][3];
+        fT[0][0] = c[4]; fT[1][1] = c[5]; fT[2][2] = c[6];
+        fT[0][1] = fT[1][0] = c[7]; fT[0][2] = fT[2][0] = c[8]; fT[1][2] = fT[2][1] = c[9];
+        double g[3];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            double sj = q * p1[j];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) sj += fm[k] * p2[k][j];
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+#pragma unroll
+                for (int l = 0; l < 3; ++l) sj += fT[k][l] * d3[k][l][j];
+            g[j] = sj;
+        }
+        double Ap2[3][3];
+#pragma unroll
+        for (int x = 0; x < 3; ++x)
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+                Ap2[x][k] = A[x * 3 + 0] * p2[0][k] + A[x * 3 + 1] * p2[1][k] + A[x * 3 + 2] * p2[2][k];
+        double GT[3][3];
+#pragma unroll
+        for (int x = 0; x < 3; ++x)
+#pragma unroll
+            for (int y = 0; y < 3; ++y)
+                GT[x][y] = (Ap2[x][0] * A[y * 3 + 0] + Ap2[x][1] * A[y * 3 + 1] + Ap2[x][2] * A[y * 3 + 2]) * (1.0 / 3.0);
+        double* gq = g_q + a * 10;
+        gq[0] = fp[0][0][0];
+        gq[1] = dmu[0]; gq[2] = dmu[1]; gq[3] = dmu[2];
+        gq[4] = GT[0][0]; gq[5] = GT[1][1]; gq[6] = GT[2][2]; gq[7] = GT[0][1]; gq[8] = GT[0][2]; gq[9] = GT[1][2];
+        const double4 pp = pos[a];
+#pragma unroll
+        for (int cc = 0; cc < 3; ++cc)
+            g_pos[a * 3 + cc] = A[0 * 3 + cc] * g[0] + A[1 * 3 + cc] * g[1] + A[2 * 3 + cc] * g[2];
+        double mu[3] = {0, 0, 0}, Th[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
+        if (qmode & 1) {
+            const double* qc = Qc + a * 10;
+            mu[0] = qc[1]; mu[1] = qc[2]; mu[2] = qc[3];
+            Th[0][0] = qc[4]; Th[1][1] = qc[5]; Th[2][2] = qc[6];
+            Th[0][1] = Th[1][0] = qc[7]; Th[0][2] = Th[2][0] = qc[8]; Th[1][2] = Th[2][1] = qc[9];
+        }
+        if (qmode & 2) { mu[0] += U[a * 3]; mu[1] += U[a * 3 + 1]; mu[2] += U[a * 3 + 2]; }
+        const double r[3] = {pp.x, pp.y, pp.z};
+        double* v = vir_atom + a * 9;
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+#pragma unroll
+            for (int cc = 0; cc < 3; ++cc) {
+                double TAp = 0;
+#pragma unroll
+                for (int x = 0; x < 3; ++x) TAp += Th[j][x] * Ap2[x][cc];
+                v[j * 3 + cc] = g[j] * r[cc] + mu[j] * p1[cc] + (2.0 / 3.0) * TAp;
+            }
+    }
+}
+
 template <class R, int MODE>
 __global__ void __launch_bounds__(8 * GATHER_SITES_PER_BLOCK)
 k_gather_ml(int N, int K0, int K1, int K2, const double4* __restrict__ pos, const BoxInfo* __restrict__ boxes,
@@ -1207,22 +1327,12 @@ k_gather_ml(int N, int K0, int K1, int K2, const double4* __restrict__ pos, cons
 #pragma unroll
             for (int bb = 0; bb < ND; ++bb)
                 if (c + aa + bb < ND) fp[c][aa][bb] = group_sum(fp[c][aa][bb], 8);
+    double zw = 0;
+    if (active && lane == 0)
+        gather_site_out<R, MODE>(a, A, fp, pos, fq, Qc, U, qmode, out3, g_q, g_pos, vir_atom, e_pol, e_real, e_z, epi.f1,
+                                 zw);
     if constexpr (MODE == 2) {
         __shared__ double shz[GS / 8];
-        double zw = 0;
-        if (active && lane == 0) {
-            const double q1[3] = {fp[1][0][0], fp[0][1][0], fp[0][0][1]};
-            const double ap = e_pol < 1e-8 ? 1e-8 : e_pol;
-            const double d = DIELECTRIC / ap - 2.0 * DIELECTRIC * epi.f1;
-#pragma unroll
-            for (int c = 0; c < 3; ++c) {
-                const double dm = A[c * 3 + 0] * q1[0] + A[c * 3 + 1] * q1[1] + A[c * 3 + 2] * q1[2];
-                const double zv = e_z[c];
-                const double wv = e_real[c] + dm + d * zv;
-                out3[a * 3 + c] = wv;
-                zw += zv * wv;
-            }
-        }
         zw = group_sum(zw, 64);
         if ((threadIdx.x & 63) == 0) shz[threadIdx.x >> 6] = zw;
         __syncthreads();
@@ -1232,101 +1342,6 @@ k_gather_ml(int N, int K0, int K1, int K2, const double4* __restrict__ pos, cons
             for (int w = 1; w < GS / 8; ++w) t += shz[w];
             epi.parts.zw(f)[sb] = t;
         }
-        return;
-    }
-    if (!active || lane != 0) return;
-    const double p1[3] = {fp[1][0][0], fp[0][1][0], fp[0][0][1]};
-    double dmu[3];
-#pragma unroll
-    for (int c = 0; c < 3; ++c) dmu[c] = A[c * 3 + 0] * p1[0] + A[c * 3 + 1] * p1[1] + A[c * 3 + 2] * p1[2];
-    if constexpr (MODE == 1) {
-        out3[a * 3 + 0] = dmu[0]; out3[a * 3 + 1] = dmu[1]; out3[a * 3 + 2] = dmu[2];
-        return;
-    } else {
-        double p2[3][3];
-        p2[0][0] = fp[2][0][0]; p2[1][1] = fp[0][2][0]; p2[2][2] = fp[0][0][2];
-        p2[0][1] = p2[1][0] = fp[1][1][0]; p2[0][2] = p2[2][0] = fp[1][0][1]; p2[1][2] = p2[2][1] = fp[0][1][1];
-        // third derivatives d3[j][k][l] (symmetric), from the ten independent entries
-        double d3[3][3][3];
-#pragma unroll
-        for (int j = 0; j < 3; ++j)
-#pragma unroll
-            for (int k = 0; k < 3; ++k)
-#pragma unroll
-                for (int l = 0; l < 3; ++l) {
-                    const int ox = (j == 0) + (k == 0) + (l == 0);
-                    const int oy = (j == 1) + (k == 1) + (l == 1);
-                    const int oz = (j == 2) + (k == 2) + (l == 2);
-                    double v = 0;
-                    if (ox == 3) v = fp[3][0][0];
-                    else if (oy == 3) v = fp[0][3][0];
-                    else if (oz == 3) v = fp[0][0][3];
-                    else if (ox == 2 && oy == 1) v = fp[2][1][0];
-                    else if (ox == 2 && oz == 1) v = fp[2][0][1];
-                    else if (oy == 2 && ox == 1) v = fp[1][2][0];
-                    else if (oy == 2 && oz == 1) v = fp[0][2][1];
-                    else if (oz == 2 && ox == 1) v = fp[1][0][2];
-                    else if (oz == 2 && oy == 1) v = fp[0][1][2];
-                    else v = fp[1][1][1];
-                    d3[j][k][l] = v;
-                }
-        const R* c = fq + a * 10;
-        const double q = (double)c[0];
-        const double fm[3] = {(double)c[1], (double)c[2], (double)c[3]};
-        double fT[3][3];
-        fT[0][0] = c[4]; fT[1][1] = c[5]; fT[2][2] = c[6];
-        fT[0][1] = fT[1][0] = c[7]; fT[0][2] = fT[2][0] = c[8]; fT[1][2] = fT[2][1] = c[9];
-        double g[3];
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            double sj = q * p1[j];
-#pragma unroll
-            for (int k = 0; k < 3; ++k) sj += fm[k] * p2[k][j];
-#pragma unroll
-            for (int k = 0; k < 3; ++k)
-#pragma unroll
-                for (int l = 0; l < 3; ++l) sj += fT[k][l] * d3[k][l][j];
-            g[j] = sj;
-        }
-        double Ap2[3][3];
-#pragma unroll
-        for (int x = 0; x < 3; ++x)
-#pragma unroll
-            for (int k = 0; k < 3; ++k)
-                Ap2[x][k] = A[x * 3 + 0] * p2[0][k] + A[x * 3 + 1] * p2[1][k] + A[x * 3 + 2] * p2[2][k];
-        double GT[3][3];
-#pragma unroll
-        for (int x = 0; x < 3; ++x)
-#pragma unroll
-            for (int y = 0; y < 3; ++y)
-                GT[x][y] = (Ap2[x][0] * A[y * 3 + 0] + Ap2[x][1] * A[y * 3 + 1] + Ap2[x][2] * A[y * 3 + 2]) * (1.0 / 3.0);
-        double* gq = g_q + a * 10;
-        gq[0] = fp[0][0][0];
-        gq[1] = dmu[0]; gq[2] = dmu[1]; gq[3] = dmu[2];
-        gq[4] = GT[0][0]; gq[5] = GT[1][1]; gq[6] = GT[2][2]; gq[7] = GT[0][1]; gq[8] = GT[0][2]; gq[9] = GT[1][2];
-        const double4 pp = pos[a];
-#pragma unroll
-        for (int cc = 0; cc < 3; ++cc)
-            g_pos[a * 3 + cc] = A[0 * 3 + cc] * g[0] + A[1 * 3 + cc] * g[1] + A[2 * 3 + cc] * g[2];
-        double mu[3] = {0, 0, 0}, Th[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
-        if (qmode & 1) {
-            const double* qc = Qc + a * 10;
-            mu[0] = qc[1]; mu[1] = qc[2]; mu[2] = qc[3];
-            Th[0][0] = qc[4]; Th[1][1] = qc[5]; Th[2][2] = qc[6];
-            Th[0][1] = Th[1][0] = qc[7]; Th[0][2] = Th[2][0] = qc[8]; Th[1][2] = Th[2][1] = qc[9];
-        }
-        if (qmode & 2) { mu[0] += U[a * 3]; mu[1] += U[a * 3 + 1]; mu[2] += U[a * 3 + 2]; }
-        const double r[3] = {pp.x, pp.y, pp.z};
-        double* v = vir_atom + a * 9;
-#pragma unroll
-        for (int j = 0; j < 3; ++j)
-#pragma unroll
-            for (int cc = 0; cc < 3; ++cc) {
-                double TAp = 0;
-#pragma unroll
-                for (int x = 0; x < 3; ++x) TAp += Th[j][x] * Ap2[x][cc];
-                v[j * 3 + cc] = g[j] * r[cc] + mu[j] * p1[cc] + (2.0 / 3.0) * TAp;
-            }
     }
 }
 
@@ -1360,7 +1375,7 @@ k_plane_matvec(int K0, int K1, int K2, FFTPlan plan0, FFTPlan plan1, const Cplx<
     }
     const int item = xcd_item(b - nplane_blocks, nbf * F);
     if (item >= nbf * F) return;
-    real_matvec_body<double, double, PLANE_THREADS>(item, N, nbf, cap, pos, boxes, nbr, ncnt, pcoef, v, out, skip);
+    real_matvec_body<double, double>(PLANE_THREADS, item, N, nbf, cap, pos, boxes, nbr, ncnt, pcoef, v, out, skip);
 }
 
 }  // namespace admp

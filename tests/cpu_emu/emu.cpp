@@ -133,24 +133,11 @@ void end_kernel() {
     g_smem_ptr = nullptr;
 }
 
-void run_block(void (*entry)(void*), void* arg, unsigned bx, unsigned by, unsigned bz) {
-    g_entry = entry;
-    g_arg = arg;
-    g_b = {bx, by, bz};
-    const unsigned n = g_bd.x * g_bd.y * g_bd.z;
-    while (F.size() < n) {
-        Fiber* f = new Fiber();
-        f->stack = (char*)malloc(STK);
-        F.push_back(f);
-    }
-    for (unsigned t = 0; t < n; ++t) {
-        Fiber* f = F[t];
-        f->t = {t % g_bd.x, (t / g_bd.x) % g_bd.y, t / (g_bd.x * g_bd.y)};
-        f->state = 0;
-        f->started = false;
-    }
+// runs the fibres [w0, w1) of one wavefront, resolving its wave operations, until
+// every one is at a barrier or done
+static void run_wave(unsigned w0, unsigned w1, unsigned bx, unsigned by, unsigned bz) {
     for (;;) {
-        for (unsigned t = 0; t < n; ++t) {
+        for (unsigned t = w0; t < w1; ++t) {
             Fiber* f = F[t];
             if (f->state != 0) continue;
             g_cur = f;
@@ -169,63 +156,91 @@ void run_block(void (*entry)(void*), void* arg, unsigned bx, unsigned by, unsign
                 }
             }
         }
-        // every fibre is at a barrier, a wave operation or done
-        unsigned done = 0, bar = 0, wop = 0;
-        for (unsigned t = 0; t < n; ++t) {
-            const int s = F[t]->state;
-            done += s == 3; bar += s == 1; wop += s == 2;
+        int kind = -1;
+        bool any = false, mixed = false;
+        for (unsigned t = w0; t < w1; ++t) {
+            Fiber* f = F[t];
+            if (f->state == 2) {
+                if (kind >= 0 && f->kind != kind) mixed = true;
+                kind = f->kind;
+                any = true;
+            } else if (f->state == 1) {
+                mixed = true;
+            }
         }
-        if (done == n) break;
-        if (wop) {
-            for (unsigned w0 = 0; w0 < n; w0 += 64) {
-                const unsigned w1 = std::min(n, w0 + 64);
-                int kind = -1;
-                bool any = false, mixed = false;
-                for (unsigned t = w0; t < w1; ++t) {
-                    Fiber* f = F[t];
-                    if (f->state == 2) {
-                        if (kind >= 0 && f->kind != kind) mixed = true;
-                        kind = f->kind;
-                        any = true;
-                    } else if (f->state == 1) {
-                        mixed = true;
-                    }
-                }
-                if (!any) continue;
-                if (mixed) {
-                    fprintf(stderr, "EMU ERROR: divergent wave operation in kernel %s block (%u,%u,%u)\n", g_name, bx,
-                            by, bz);
+        if (!any) return;
+        if (mixed) {
+            fprintf(stderr, "EMU ERROR: divergent wave operation in kernel %s block (%u,%u,%u)\n", g_name, bx,
+                    by, bz);
+            _exit(87);
+        }
+        if (kind == 5) {
+            MmaF64* m[64];
+            for (unsigned l = 0; l < 64; ++l) {
+                if (w0 + l >= w1 || F[w0 + l]->state != 2) {
+                    fprintf(stderr, "EMU ERROR: matrix product without a full wavefront in kernel %s\n", g_name);
                     _exit(87);
                 }
-                unsigned long long ball = 0;
-                for (unsigned t = w0; t < w1; ++t)
-                    if (F[t]->state == 2 && F[t]->val) ball |= 1ull << (t - w0);
-                for (unsigned t = w0; t < w1; ++t) {
-                    Fiber* f = F[t];
-                    if (f->state != 2) continue;
-                    const unsigned l = t - w0;
-                    const int wd = f->width;
-                    const unsigned base = l & ~(unsigned)(wd - 1);
-                    long long r = f->val;
-                    auto get = [&](unsigned src, long long own) -> long long {
-                        const unsigned ts = w0 + src;
-                        if (ts < w1 && F[ts]->state == 2) return F[ts]->val;
-                        return own;
-                    };
-                    if (kind == 0) r = get(base + ((unsigned)f->arg & (unsigned)(wd - 1)), f->val);
-                    else if (kind == 1) {
-                        const unsigned src = l ^ (unsigned)f->arg;
-                        r = ((src & ~(unsigned)(wd - 1)) == base) ? get(src, f->val) : f->val;
-                    } else if (kind == 2) r = (l - base) >= (unsigned)f->arg ? get(l - f->arg, f->val) : f->val;
-                    else if (kind == 3) r = (long long)ball;
-                    else if (kind == 4) r = get((unsigned)f->arg, 0);
-                    f->res = r;
-                }
-                for (unsigned t = w0; t < w1; ++t)
-                    if (F[t]->state == 2) F[t]->state = 0;
+                m[l] = reinterpret_cast<MmaF64*>((intptr_t)F[w0 + l]->val);
             }
-            continue;
+            for (unsigned l = 0; l < 64; ++l)
+                for (unsigned r = 0; r < 4; ++r) {
+                    double d = m[l]->c[r];
+                    for (unsigned k = 0; k < 4; ++k) d += m[4 * r + l / 16 + 16 * k]->a * m[l % 16 + 16 * k]->b;
+                    m[l]->d[r] = d;
+                }
         }
+        unsigned long long ball = 0;
+        for (unsigned t = w0; t < w1; ++t)
+            if (F[t]->state == 2 && F[t]->val) ball |= 1ull << (t - w0);
+        for (unsigned t = w0; t < w1; ++t) {
+            Fiber* f = F[t];
+            if (f->state != 2) continue;
+            const unsigned l = t - w0;
+            const int wd = f->width;
+            const unsigned base = l & ~(unsigned)(wd - 1);
+            long long r = f->val;
+            auto get = [&](unsigned src, long long own) -> long long {
+                const unsigned ts = w0 + src;
+                if (ts < w1 && F[ts]->state == 2) return F[ts]->val;
+                return own;
+            };
+            if (kind == 0) r = get(base + ((unsigned)f->arg & (unsigned)(wd - 1)), f->val);
+            else if (kind == 1) {
+                const unsigned src = l ^ (unsigned)f->arg;
+                r = ((src & ~(unsigned)(wd - 1)) == base) ? get(src, f->val) : f->val;
+            } else if (kind == 2) r = (l - base) >= (unsigned)f->arg ? get(l - f->arg, f->val) : f->val;
+            else if (kind == 3) r = (long long)ball;
+            else if (kind == 4) r = get((unsigned)f->arg, 0);
+            f->res = r;
+        }
+        for (unsigned t = w0; t < w1; ++t)
+            if (F[t]->state == 2) F[t]->state = 0;
+    }
+}
+
+void run_block(void (*entry)(void*), void* arg, unsigned bx, unsigned by, unsigned bz) {
+    g_entry = entry;
+    g_arg = arg;
+    g_b = {bx, by, bz};
+    const unsigned n = g_bd.x * g_bd.y * g_bd.z;
+    while (F.size() < n) {
+        Fiber* f = new Fiber();
+        f->stack = (char*)malloc(STK);
+        F.push_back(f);
+    }
+    for (unsigned t = 0; t < n; ++t) {
+        Fiber* f = F[t];
+        f->t = {t % g_bd.x, (t / g_bd.x) % g_bd.y, t / (g_bd.x * g_bd.y)};
+        f->state = 0;
+        f->started = false;
+    }
+    for (;;) {
+        // each wavefront runs until all its fibres are at a barrier or done
+        for (unsigned w0 = 0; w0 < n; w0 += 64) run_wave(w0, std::min(n, w0 + 64), bx, by, bz);
+        unsigned done = 0;
+        for (unsigned t = 0; t < n; ++t) done += F[t]->state == 3;
+        if (done == n) break;
         for (unsigned t = 0; t < n; ++t)
             if (F[t]->state == 1) F[t]->state = 0;
     }

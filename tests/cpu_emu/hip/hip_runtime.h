@@ -9,6 +9,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <unistd.h>
 #include <tuple>
 #include <type_traits>
 #include <utility>
@@ -46,7 +47,7 @@ const uint3e& bidx();
 const uint3e& bdim();
 const uint3e& gdim();
 void syncthreads();
-long long wave_op(int kind, long long v, int arg, int width);  // 0 shfl, 1 xor, 2 up, 3 ballot, 4 readlane
+long long wave_op(int kind, long long v, int arg, int width);  // 0 shfl, 1 xor, 2 up, 3 ballot, 4 readlane, 5 matrix product
 void* dyn_smem();
 void begin_kernel(const char* name, dim3 g, dim3 b, size_t smem);
 void run_block(void (*entry)(void*), void* arg, unsigned bx, unsigned by, unsigned bz);
@@ -73,6 +74,30 @@ template <class T> inline T __shfl_up(T v, unsigned delta, int width = 64) {
 }
 inline unsigned long long __ballot(int pred) { return (unsigned long long)emu::wave_op(3, pred ? 1 : 0, 0, 64); }
 inline int __builtin_amdgcn_readlane(int v, int lane) { return (int)emu::wave_op(4, v, lane, 64); }
+// matrix product of a wavefront: register r of lane l holds row 4 r + l / 16,
+// column l % 16 of D = A B + C (A: row l % 16, column l / 16; B: row l / 16, column l % 16)
+typedef double emu_d4 __attribute__((vector_size(32)));
+namespace emu {
+struct MmaF64 { double a, b, c[4], d[4]; };
+}
+inline emu_d4 __builtin_amdgcn_mfma_f64_16x16x4f64(double a, double b, emu_d4 c, int, int, int) {
+    emu::MmaF64 m{a, b, {c[0], c[1], c[2], c[3]}, {0, 0, 0, 0}};
+    emu::wave_op(5, (long long)(intptr_t)&m, 0, 64);
+    return emu_d4{m.d[0], m.d[1], m.d[2], m.d[3]};
+}
+// accesses of a wavefront's lanes to LDS before it are visible to the others after it
+inline void __builtin_amdgcn_wave_barrier() { emu::wave_op(3, 0, 0, 64); }
+inline int __builtin_amdgcn_readfirstlane(int v) { return (int)emu::wave_op(4, v, 0, 64); }
+// quad_perm [1, 0, 3, 2] (0xB1), quad_perm [2, 3, 0, 1] (0x4E), row_half_mirror (0x141:
+// the eight lanes of a half row in reverse)
+inline int __builtin_amdgcn_mov_dpp(int v, int ctrl, int, int, bool) {
+    const int m = ctrl == 0xB1 ? 1 : ctrl == 0x4E ? 2 : ctrl == 0x141 ? 7 : 0;
+    if (!m) { fprintf(stderr, "EMU ERROR: dpp control %#x\n", ctrl); _exit(87); }
+    return (int)emu::wave_op(1, v, m, 64);
+}
+inline long long __double_as_longlong(double v) { return emu::to_bits(v); }
+inline double __longlong_as_double(long long v) { return emu::from_bits<double>(v); }
+#define __builtin_amdgcn_fence(order, scope) ((void)0)
 inline int __popcll(unsigned long long v) { return __builtin_popcountll(v); }
 inline int __ffsll(long long v) { return __builtin_ffsll(v); }
 template <class T> inline T atomicAdd(T* p, T v) { T o = *p; *p = o + v; return o; }

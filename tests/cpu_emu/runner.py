@@ -439,6 +439,9 @@ if __name__ == "__main__":
     patch_engine(lib)
     if case == "grid":
         out = grid(prec, tuple(int(k) for k in sys.argv[4].split(",")))
+    elif case == "polar_grid":
+        from tests.systems import polar_grid
+        out = {k: _lst(v) for k, v in polar_grid(tuple(int(k) for k in sys.argv[4].split(",")), "cpu").items()}
     elif case == "waters":
         out = waters(prec, int(sys.argv[4]))
     elif case == "frames" and len(sys.argv) > 4:

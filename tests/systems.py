@@ -296,6 +296,49 @@ def library_pme(pos, box, axis_types, axis_idx, bonded, Q, pol, thole, scales, r
     return out
 
 
+# a row tile of the matrix-core transforms holds 16 outputs of the half spectrum: 31 | 32 and
+# 63 | 64 points are one row tile | two and two | three; odd and even, primes, the shortest and
+# the longest axes, axes of a tile that is only part full, and planes past the LDS (y and x
+# lines in passes of their own)
+MATRIX_GRIDS = [(9, 10, 11), (31, 32, 16), (17, 33, 31), (12, 63, 64), (13, 9, 128), (97, 101, 10), (128, 127, 9)]
+
+
+def polar_grid(K, device):
+    """Two frames of the small box with induced dipoles on a given grid."""
+    from dmff_amd.admp.engine import Engine
+    from dmff_amd.admp.pme import setup_ewald_parameters
+    s, pos, box = small_water_box()
+    rng = np.random.default_rng(17)
+    P = np.stack([pos, pos + rng.normal(0, 0.02, pos.shape)])
+    B = np.stack([box, box * 1.01])
+    kappa = setup_ewald_parameters(6.0, 5e-4, box)[0]
+    eng = Engine(len(pos), 2, True, True, kappa, K, 6.0, n_frames=2, device=device)
+    eng.set_topology(s.axis_types, s.axis_idx, s.bonded)
+    eng.build_neighbors(P, B)
+    E, g, U, info = eng.compute(P, B, s.pme.Q_local[s.map_atomtype], s.pme.pol[s.map_poltype],
+                                s.pme.thole[s.map_poltype], s.pme.mScales, s.pme.pScales, s.pme.dScales,
+                                solver="pcg", tol=1e-11, maxiter=200, want_grad=True)
+    out = {"E": E, "U": U, "pos": g["pos"], "box": g["box"], "Q": g["Q"]}
+    return {k: v.cpu().numpy() for k, v in out.items()}
+
+
+def polar_grid_oracle(K):
+    """Frame 0 of polar_grid by the oracle."""
+    import torch
+    from oracle import admp_oracle as O
+    s, pos, box = small_water_box()
+    f = O.ADMPPmeForce(box, s.axis_types, s.axis_idx, 6.0, 5e-4, 2, True, True, None)
+    f.K = tuple(K)
+    T = lambda x: torch.tensor(np.asarray(x, dtype=np.float64), requires_grad=True)
+    p, b, q = T(pos), T(box), T(s.pme.Q_local[s.map_atomtype])
+    e, aux = f.get_energy(p, b, reference_pairs(pos, box, 6.0, s.bonded), q, T(s.pme.pol[s.map_poltype]),
+                          T(s.pme.thole[s.map_poltype]), s.pme.mScales, s.pme.pScales, s.pme.dScales, solver="cg",
+                          tol=1e-10, aux={})
+    gp, gb, gq = torch.autograd.grad(e, (p, b, q))
+    return {"E": e.detach().numpy(), "U": aux["U_ind"].detach().numpy() * 10.0, "pos": gp.numpy(), "box": gb.numpy(),
+            "Q": gq.numpy()}
+
+
 def rel_err(a, b, floor=1e-6):
     a = np.asarray(a, dtype=np.float64).ravel()
     b = np.asarray(b, dtype=np.float64).ravel()

@@ -22,7 +22,7 @@ import pytest
 import torch
 
 from oracle import admp_oracle as O
-from tests.systems import reference_pairs, small_water_box
+from tests.systems import MATRIX_GRIDS, reference_pairs, small_water_box
 from tests.test_gpu_parity import compare, oracle_eval, rel_rms
 
 REPO = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -160,6 +160,19 @@ def test_grid_paths(emu_lib, K, prec):
     etol, ftol = (1e-9, 1e-7) if prec == "fp64" else (2e-5, 1e-4)
     assert abs(r["E"] - float(e)) < etol * abs(float(e))
     assert rel_rms(r["pos"], gp.numpy()) < ftol
+
+
+@pytest.mark.parametrize("K", MATRIX_GRIDS)
+def test_matrix_core_grids_equal_radix_path(emu_lib, K):
+    """The FP64 spread, transforms and gather on the matrix cores against the radix path
+    at the edges of their tiles.  Both round in 64 bits: a transform of n points is off by
+    about log2(n) eps on the radix path and by sqrt(n) eps as a dense sum, 3e-15 relative to
+    the largest value of the grid; the solve (condition number below 100, residual 1e-11)
+    leaves 1e-9."""
+    a, b = (run(emu_lib, "polar_grid", "fp64", ",".join(str(k) for k in K), extra_env=e)
+            for e in (None, {"ADMP_SPREAD": "cw"}))
+    for key in a:
+        assert rel_rms(a[key], b[key]) < 1e-9, key
 
 
 def test_water_box_several_solver_blocks(emu_lib):
