@@ -121,15 +121,280 @@ struct PairParams {
 };
 
 // ---------------------------------------------------------------------------
+// The FP64 final pass (the same terms as the general body of k_real_final below).
+// Bound by FP64 issue and by the latency of the neighbours' records, so it is laid out
+// for wavefronts in flight: the general body holds 320 registers in FP64 (one wavefront
+// per SIMD).  Here a pair takes three steps with few values between them: the pair's
+// invariants, from both records; the radial functions, of which the combinations that the
+// gradients need stay; the gradients, which read the records again (from L2, and the own site's from LDS).
+// The virial differs from zero only for pairs across the boundary: its sums stay in LDS.
+// pair_step() ends a step for the compiler, which would otherwise load early and hold.
+// 225 registers' worth of values instead of 320, two wavefronts per SIMD, 753 FP64
+// instructions per pair instead of 906: 180 -> 155 us at 12,288 sites (90 neighbours each),
+// 10.4 -> 7.5 ms for 64 such frames.  Forcing three wavefronts spills 80 registers: 16 ms.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ void pair_step(int& j) {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" : "+v"(j) : : "memory");   // an index it cannot know: no record is kept for the next step
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+template <bool LPOL>
+__device__ __forceinline__ void real_final64(int N, int cap, const double4* __restrict__ pos, const BoxInfo* __restrict__ boxes,
+                                             const double* __restrict__ site, const int* __restrict__ nbr,
+                                             const int* __restrict__ ncnt, const PairParams& pp, double* __restrict__ e_atom,
+                                             double* __restrict__ g_pos, double* __restrict__ g_q, double* __restrict__ vir_atom,
+                                             double* __restrict__ g_pol, double* __restrict__ g_thole) {
+    __shared__ double own[PAIR_BLOCK / TPA][SITE + 1];   // the block's own sites
+    __shared__ double vl[9][PAIR_BLOCK];
+    const int f = blockIdx.y;
+    const int gt = blockIdx.x * PAIR_BLOCK + threadIdx.x;
+    const int i = gt / TPA, sub = gt % TPA;
+    const bool active = i < N;
+    const int ii = active ? i : 0;
+    const BoxInfo& bx = boxes[f];
+    const size_t fo = (size_t)f * N;
+    double* I = own[threadIdx.x / TPA];
+    I[sub] = site[(fo + ii) * SITE + sub];
+    static_assert(SITE == TPA, "one lane per word of the own record");
+    const int vt = threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < 9; ++k) vl[k][vt] = 0;
+    const double4 pi_ = pos[fo + ii];
+    const double kap = pp.kappa, k1 = K1_INV;
+    __syncthreads();
+    double E = 0, gx = 0, gy = 0, gz = 0, gq = 0, gmx = 0, gmy = 0, gmz = 0;
+    double gTxx = 0, gTyy = 0, gTzz = 0, gTxy = 0, gTxz = 0, gTyz = 0, gpol = 0, gth = 0;
+    const int cnt = active ? ncnt[fo + ii] : 0;
+    const int* nl = nbr + (fo + ii) * (size_t)cap;
+    int w = sub < cnt ? nl[sub] : 0;
+#pragma unroll 1
+    for (int k = sub; k < cnt; k += TPA) {
+        int j = w & NB_MASK;
+        const int sidx = scale_index(w >> NB_SHIFT, pp.nscale);
+        if (k + TPA < cnt) w = nl[k + TPA];
+        const double4 pj = pos[fo + j];
+        const double* J = site + (fo + j) * SITE;
+        double dx = pi_.x - pj.x, dy = pi_.y - pj.y, dz = pi_.z - pj.z, n0, n1, n2;
+        pbc_shift(bx, dx, dy, dz, n0, n1, n2);
+        const double r = sqrt(dx * dx + dy * dy + dz * dz), rinv = 1.0 / r;
+        const double zx = dx * rinv, zy = dy * rinv, zz = dz * rinv;
+        // ---- invariants ----
+        double p0, p1, p2, p3, p4, p5, p6, p7, p8, p9, u0 = 0, u1 = 0, u2 = 0, u3 = 0, u4 = 0, u5 = 0, u6 = 0;
+        {
+            const double qI = I[0], mIx = I[1], mIy = I[2], mIz_ = I[3], qJ = J[0], mJx = J[1], mJy = J[2], mJz_ = J[3];
+            const double tIx = I[4] * zx + I[7] * zy + I[8] * zz, tIy = I[7] * zx + I[5] * zy + I[9] * zz;
+            const double tIz = I[8] * zx + I[9] * zy + I[6] * zz;
+            const double tJx = J[4] * zx + J[7] * zy + J[8] * zz, tJy = J[7] * zx + J[5] * zy + J[9] * zz;
+            const double tJz = J[8] * zx + J[9] * zy + J[6] * zz;
+            const double mIz = mIx * zx + mIy * zy + mIz_ * zz, mJz = mJx * zx + mJy * zy + mJz_ * zz;
+            const double zzI = tIx * zx + tIy * zy + tIz * zz, zzJ = tJx * zx + tJy * zy + tJz * zz;
+            const double tImJ = tIx * mJx + tIy * mJy + tIz * mJz_, tJmI = tJx * mIx + tJy * mIy + tJz * mIz_;
+            const double tItJ = tIx * tJx + tIy * tJy + tIz * tJz;
+            const double ThTh = I[4] * J[4] + I[5] * J[5] + I[6] * J[6] + 2.0 * (I[7] * J[7] + I[8] * J[8] + I[9] * J[9]);
+            p0 = qI * qJ;
+            p1 = qI * mJz - qJ * mIz;
+            p2 = mIz * mJz;
+            p3 = mIx * mJx + mIy * mJy + mIz_ * mJz_ - p2;
+            p4 = qI * zzJ + qJ * zzI;
+            p5 = zzI * mJz - zzJ * mIz;
+            p6 = k1 * ((tImJ - zzI * mJz) - (tJmI - zzJ * mIz));
+            p7 = zzI * zzJ;
+            p8 = (4.0 / 3.0) * (tItJ - p7);
+            p9 = (2.0 / 3.0) * ThTh + (1.0 / 3.0) * p7 - (4.0 / 3.0) * tItJ;
+            if constexpr (LPOL) {
+                const double UIx = I[13], UIy = I[14], UIz = I[15], UJx = J[13], UJy = J[14], UJz = J[15];
+                const double uIz = UIx * zx + UIy * zy + UIz * zz, uJz = UJx * zx + UJy * zy + UJz * zz;
+                u0 = qI * uJz - qJ * uIz;
+                u1 = mJz * uIz + mIz * uJz;
+                u2 = (mJx * UIx + mJy * UIy + mJz_ * UIz - mJz * uIz) + (mIx * UJx + mIy * UJy + mIz_ * UJz - mIz * uJz);
+                u3 = zzI * uJz - zzJ * uIz;
+                u4 = k1 * ((tIx * UJx + tIy * UJy + tIz * UJz - zzI * uJz) - (tJx * UIx + tJy * UIy + tJz * UIz - zzJ * uIz));
+                u5 = uIz * uJz;
+                u6 = UIx * UJx + UIy * UJy + UIz * UJz - u5;
+            }
+        }
+        pair_step(j);
+        J = site + (fo + j) * SITE;
+        // ---- radial functions ----
+        // Every coefficient is D / r^n times (scale + b) and terms in x = kappa r, so the energy
+        // S1 + .. + S5, one sum per power of 1/r, has the slope -(S1 + 2 S2 + .. + 5 S5) / r plus
+        // that of b and the x terms at fixed r^-n, in which the erf cancels: a polynomial in x
+        // times exp(-x^2), the same for permanent and induced terms.
+        double dEdr, cc, cd, ddm, dd1, cq, dq0, ktm, qq0, qq1, qq2;   // ddm = dd0 - dd1, ktm = k1 dq1
+        double cud = 0, dudm = 0, dud1 = 0, udq0 = 0, ktu = 0, udm = 0;
+        {
+            const double ms = pp.ms[sidx];
+            const double x = kap * r, x2 = x * x;
+            const double X = TWO_OVER_SQRT_PI * exp(-x2);
+            const double Y1 = x * X, Y3 = x2 * Y1, Y5 = x2 * Y3;
+            const double b2 = Y1 - erf(x), b3 = b2 + (2.0 / 3.0) * Y3, b4 = b3 + (4.0 / 15.0) * Y5;
+            const double P1 = DIELECTRIC * rinv, P2 = P1 * rinv, P3 = P2 * rinv, P4 = P3 * rinv, P5 = P4 * rinv;
+            const double q1 = p1 + u0, q2 = p2 + u1 + u5, q3 = p3 + u2 + u6, q5 = p5 + u3, q6 = p6 + u4;
+            const double kap2 = kap * kap;
+            dEdr = kap * X * P1 *
+                   (-p0 - 2.0 * kap * x * q1 + kap2 * (x2 * (4.0 * q2 - (4.0 / 3.0) * p4) - 2.0 * (q2 + q3)) +
+                    kap2 * kap * x * ((8.0 / 3.0) * (1.0 - x2) * q5 + (4.0 / SQRT3) * q6) +
+                    kap2 * kap2 * (x2 * ((32.0 / 9.0) * p7 + (8.0 / 3.0) * p8 - (16.0 / 9.0) * x2 * p7) -
+                                   (4.0 / 3.0) * (p7 + p8 + p9)));
+            cc = P1 * (ms + b2 - Y1);
+            cd = P2 * (ms + b2);
+            const double A3 = ms + b3, A4 = ms + b4;
+            ddm = -2.0 * P3 * (A3 + (1.0 / 3.0) * Y3);
+            dd1 = P3 * (A3 - (2.0 / 3.0) * Y3);
+            cq = P3 * A3;
+            dq0 = P4 * (3.0 * A3 + (4.0 / 3.0) * Y5);
+            const double dq1 = -SQRT3 * P4 * A3;
+            qq0 = P5 * (6.0 * A4 + (4.0 / 45.0) * (10.0 * x2 - 3.0) * Y5);
+            qq1 = -P5 * (4.0 * A4 + (4.0 / 15.0) * Y5);
+            qq2 = P5 * (A4 - (4.0 / 15.0) * Y5);
+            const double S1 = cc * p0, S5 = qq0 * p7 + qq1 * p8 + qq2 * p9;
+            double S2 = cd * p1, S3 = ddm * p2 + dd1 * p3 + cq * p4, S4 = dq0 * p5 + dq1 * p6;
+            ddm -= dd1;
+            ktm = k1 * dq1;
+            if constexpr (LPOL) {
+                const double ps = pp.ps[sidx], dsc = pp.ds[sidx];
+                // Thole width and argument (pme.py:793-801)
+                const double a = ps > 0.0 ? 5.0 : I[11] + J[11];
+                const double aa = I[10] * J[10];
+                const bool dmp_cl = aa < 1e-8;
+                const double idmp = 1.0 / (dmp_cl ? 1e-8 : aa);
+                double u = r * idmp;
+                const bool u_cl = !(u < 1e8);
+                if (u_cl) u = 1e8;
+                const double au = a * u;
+                Thole<double> th;
+                thole_f<double>(au, th);
+                const double psc = ps * th.c, dscc = dsc * th.c;
+                cud = P2 * (psc + b2);
+                dudm = -2.0 * P3 * (ps * th.d0 + b3 + (1.0 / 3.0) * Y3);
+                dud1 = P3 * (psc + b3 - (2.0 / 3.0) * Y3);
+                udq0 = P4 * (3.0 * (ps * th.q0 + b3) + (4.0 / 3.0) * Y5);
+                const double udq1 = -SQRT3 * P4 * (ps * th.q1 + b3);
+                udm = -2.0 * P3 * (dsc * th.d0 + b3 + (1.0 / 3.0) * Y3);
+                const double ud1 = P3 * (dscc + b3 - (2.0 / 3.0) * Y3);
+                S2 += cud * u0;
+                S3 += dudm * u1 + dud1 * u2 + udm * u5 + ud1 * u6;
+                S4 += udq0 * u3 + udq1 * u4;
+                dudm -= dud1;
+                udm -= ud1;
+                ktu = k1 * udq1;
+                // dE/dau through the Thole functions
+                const double dEdau = P2 * ps * u0 * th.dc - 2.0 * P3 * (ps * u1 + dsc * u5) * th.dd0 +
+                                     P3 * (ps * u2 + dsc * u6) * th.dc + P4 * ps * (3.0 * u3 * th.dq0 - SQRT3 * u4 * th.dq1);
+                if (!u_cl) dEdr += dEdau * a * idmp;
+                // d au / d alpha_I = -au aa / (6 alpha_I dmp): the division by 6 alpha_I follows the loop
+                gpol -= (dmp_cl || u_cl) ? 0.0 : dEdau * au * idmp * aa;
+                gth += ps > 0.0 ? 0.0 : dEdau * u;
+            }
+            E += S1 + S2 + S3 + S4 + S5;
+            dEdr -= rinv * (S1 + 2.0 * S2 + 3.0 * S3 + 4.0 * S4 + 5.0 * S5);
+        }
+        pair_step(j);
+        J = site + (fo + j) * SITE;
+        // ---- gradients ----
+        const double qI = I[0], mIx = I[1], mIy = I[2], mIz_ = I[3], qJ = J[0], mJx = J[1], mJy = J[2], mJz_ = J[3];
+        const double tIx = I[4] * zx + I[7] * zy + I[8] * zz, tIy = I[7] * zx + I[5] * zy + I[9] * zz;
+        const double tIz = I[8] * zx + I[9] * zy + I[6] * zz;
+        const double tJx = J[4] * zx + J[7] * zy + J[8] * zz, tJy = J[7] * zx + J[5] * zy + J[9] * zz;
+        const double tJz = J[8] * zx + J[9] * zy + J[6] * zz;
+        const double mIz = mIx * zx + mIy * zy + mIz_ * zz, mJz = mJx * zx + mJy * zy + mJz_ * zz;
+        const double zzI = tIx * zx + tIy * zy + tIz * zz, zzJ = tJx * zx + tJy * zy + tJz * zz;
+        const double etItJ = (4.0 / 3.0) * (qq1 - qq2), eThTh = (2.0 / 3.0) * qq2;
+        const double czz = qq0 - (4.0 / 3.0) * qq1 + (1.0 / 3.0) * qq2, kd = ktm - dq0;
+        double e_mIz = -cd * qJ + ddm * mJz + kd * zzJ, e_mJz = cd * qI + ddm * mIz - kd * zzI;
+        double e_zzI = cq * qJ - kd * mJz + czz * zzJ, e_zzJ = cq * qI + kd * mIz + czz * zzI;
+        // the vectors multiplied by Theta_I (a) and Theta_J (b) in dE/dz; sym(z a) enters
+        // dE/dTheta_I
+        double ax = ktm * mJx + etItJ * tJx, ay = ktm * mJy + etItJ * tJy, az = ktm * mJz_ + etItJ * tJz;
+        double bx_ = etItJ * tIx - ktm * mIx, by_ = etItJ * tIy - ktm * mIy, bz_ = etItJ * tIz - ktm * mIz_;
+        double gqI = cc * qJ + cd * mJz + cq * zzJ;
+        double hx = dd1 * mJx - ktm * tJx, hy = dd1 * mJy - ktm * tJy, hz = dd1 * mJz_ - ktm * tJz;
+        double Zx = 0, Zy = 0, Zz = 0;
+        if constexpr (LPOL) {
+            const double UIx = I[13], UIy = I[14], UIz = I[15], UJx = J[13], UJy = J[14], UJz = J[15];
+            const double uIz = UIx * zx + UIy * zy + UIz * zz, uJz = UJx * zx + UJy * zy + UJz * zz;
+            const double kdu = ktu - udq0;
+            e_mIz += dudm * uJz;
+            e_mJz += dudm * uIz;
+            e_zzI -= kdu * uJz;
+            e_zzJ += kdu * uIz;
+            const double e_uIz = -cud * qJ + dudm * mJz + kdu * zzJ + udm * uJz;
+            const double e_uJz = cud * qI + dudm * mIz - kdu * zzI + udm * uIz;
+            gqI += cud * uJz;
+            hx += dud1 * UJx; hy += dud1 * UJy; hz += dud1 * UJz;
+            ax += ktu * UJx; ay += ktu * UJy; az += ktu * UJz;
+            bx_ -= ktu * UIx; by_ -= ktu * UIy; bz_ -= ktu * UIz;
+            Zx = e_uIz * UIx + e_uJz * UJx;
+            Zy = e_uIz * UIy + e_uJz * UJy;
+            Zz = e_uIz * UIz + e_uJz * UJz;
+        }
+        gq += gqI;
+        gmx += hx + e_mIz * zx; gmy += hy + e_mIz * zy; gmz += hz + e_mIz * zz;
+        // dE/dTheta_I = e_zzI z z^T + sym(z a^T) + e_ThTh Theta_J   (matrix entries)
+        gTxx += e_zzI * zx * zx + zx * ax + eThTh * J[4];
+        gTyy += e_zzI * zy * zy + zy * ay + eThTh * J[5];
+        gTzz += e_zzI * zz * zz + zz * az + eThTh * J[6];
+        gTxy += e_zzI * zx * zy + 0.5 * (zx * ay + zy * ax) + eThTh * J[7];
+        gTxz += e_zzI * zx * zz + 0.5 * (zx * az + zz * ax) + eThTh * J[8];
+        gTyz += e_zzI * zy * zz + 0.5 * (zy * az + zz * ay) + eThTh * J[9];
+        // dE/dz: Theta_I a + Theta_J b, and 2 e_zz t = Theta (2 e_zz z)
+        ax += 2.0 * e_zzI * zx; ay += 2.0 * e_zzI * zy; az += 2.0 * e_zzI * zz;
+        bx_ += 2.0 * e_zzJ * zx; by_ += 2.0 * e_zzJ * zy; bz_ += 2.0 * e_zzJ * zz;
+        Zx += e_mIz * mIx + e_mJz * mJx + I[4] * ax + I[7] * ay + I[8] * az + J[4] * bx_ + J[7] * by_ + J[8] * bz_;
+        Zy += e_mIz * mIy + e_mJz * mJy + I[7] * ax + I[5] * ay + I[9] * az + J[7] * bx_ + J[5] * by_ + J[9] * bz_;
+        Zz += e_mIz * mIz_ + e_mJz * mJz_ + I[8] * ax + I[9] * ay + I[6] * az + J[8] * bx_ + J[9] * by_ + J[6] * bz_;
+        const double zZ = Zx * zx + Zy * zy + Zz * zz;
+        const double fx = dEdr * zx + (Zx - zZ * zx) * rinv;
+        const double fy = dEdr * zy + (Zy - zZ * zy) * rinv;
+        const double fz = dEdr * zz + (Zz - zZ * zz) * rinv;
+        gx += fx; gy += fy; gz += fz;
+        if (n0 != 0.0 || n1 != 0.0 || n2 != 0.0) {
+            vl[0][vt] -= n0 * fx; vl[1][vt] -= n0 * fy; vl[2][vt] -= n0 * fz;
+            vl[3][vt] -= n1 * fx; vl[4][vt] -= n1 * fy; vl[5][vt] -= n1 * fz;
+            vl[6][vt] -= n2 * fx; vl[7][vt] -= n2 * fy; vl[8][vt] -= n2 * fz;
+        }
+    }
+    E = group_sum(E, TPA);
+    gx = group_sum(gx, TPA); gy = group_sum(gy, TPA); gz = group_sum(gz, TPA);
+    gq = group_sum(gq, TPA);
+    gmx = group_sum(gmx, TPA); gmy = group_sum(gmy, TPA); gmz = group_sum(gmz, TPA);
+    gTxx = group_sum(gTxx, TPA); gTyy = group_sum(gTyy, TPA); gTzz = group_sum(gTzz, TPA);
+    gTxy = group_sum(gTxy, TPA); gTxz = group_sum(gTxz, TPA); gTyz = group_sum(gTyz, TPA);
+    if (LPOL) { gpol = group_sum(gpol, TPA); gth = group_sum(gth, TPA); }
+    const size_t a = fo + ii;
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+        const double v = group_sum(vl[k][vt], TPA);
+        if (active && sub == k) vir_atom[a * 9 + k] = 0.5 * v;
+    }
+    if (active && sub == 0) {
+        e_atom[a] = 0.5 * E;
+        g_pos[a * 3 + 0] = gx; g_pos[a * 3 + 1] = gy; g_pos[a * 3 + 2] = gz;
+        double* q = g_q + a * 10;
+        q[0] = gq; q[1] = gmx; q[2] = gmy; q[3] = gmz;
+        q[4] = gTxx; q[5] = gTyy; q[6] = gTzz; q[7] = gTxy; q[8] = gTxz; q[9] = gTyz;
+        if (LPOL) {
+            const double al = I[12];
+            g_pol[a] = al > 0.0 ? gpol / (6.0 * al) : 0.0;
+            g_thole[a] = gth;
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Final pass: energy and every gradient, U held fixed.
 // ---------------------------------------------------------------------------
 template <class R, bool LPOL>
-__global__ void __launch_bounds__(PAIR_BLOCK)
+__global__ void __launch_bounds__(PAIR_BLOCK, sizeof(R) == 8 ? 2 : 1)
 k_real_final(int N, int cap, const double4* __restrict__ pos, const BoxInfo* __restrict__ boxes,
              const R* __restrict__ site, const int* __restrict__ nbr, const int* __restrict__ ncnt,
              PairParams pp, double* __restrict__ e_atom, double* __restrict__ g_pos,
              double* __restrict__ g_q, double* __restrict__ vir_atom, double* __restrict__ g_pol,
              double* __restrict__ g_thole) {
+    if constexpr (sizeof(R) == 8) {
+        real_final64<LPOL>(N, cap, pos, boxes, site, nbr, ncnt, pp, e_atom, g_pos, g_q, vir_atom, g_pol, g_thole);
+    } else {
     const int f = blockIdx.y;
     const int gt = blockIdx.x * PAIR_BLOCK + threadIdx.x;
     const int i = gt / TPA, sub = gt % TPA;
@@ -379,6 +644,7 @@ k_real_final(int N, int cap, const double4* __restrict__ pos, const BoxInfo* __r
         v[3] = 0.5 * v10; v[4] = 0.5 * v11; v[5] = 0.5 * v12;
         v[6] = 0.5 * v20; v[7] = 0.5 * v21; v[8] = 0.5 * v22;
         if (LPOL) { g_pol[a] = gpol; g_thole[a] = gth; }
+    }
     }
 }
 

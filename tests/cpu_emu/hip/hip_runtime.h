@@ -87,6 +87,7 @@ inline emu_d4 __builtin_amdgcn_mfma_f64_16x16x4f64(double a, double b, emu_d4 c,
 }
 // accesses of a wavefront's lanes to LDS before it are visible to the others after it
 inline void __builtin_amdgcn_wave_barrier() { emu::wave_op(3, 0, 0, 64); }
+#define __builtin_amdgcn_sched_barrier(mask) ((void)0)
 inline int __builtin_amdgcn_readfirstlane(int v) { return (int)emu::wave_op(4, v, 0, 64); }
 // quad_perm [1, 0, 3, 2] (0xB1), quad_perm [2, 3, 0, 1] (0x4E), row_half_mirror (0x141:
 // the eight lanes of a half row in reverse)
