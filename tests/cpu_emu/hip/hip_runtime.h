@@ -101,6 +101,7 @@ inline double __longlong_as_double(long long v) { return emu::from_bits<double>(
 #define __builtin_amdgcn_fence(order, scope) ((void)0)
 inline int __popcll(unsigned long long v) { return __builtin_popcountll(v); }
 inline int __ffsll(long long v) { return __builtin_ffsll(v); }
+template <class T> inline T atomicCAS(T* p, T e, T v) { T o = *p; if (o == e) *p = v; return o; }
 template <class T> inline T atomicAdd(T* p, T v) { T o = *p; *p = o + v; return o; }
 inline int atomicMax(int* p, int v) { int o = *p; if (v > o) *p = v; return o; }
 inline int atomicExch(int* p, int v) { int o = *p; *p = v; return o; }

@@ -66,6 +66,31 @@ def _rel(a, b):
     return float(np.linalg.norm(a - b) / max(np.linalg.norm(b), 1e-300))
 
 
+@pytest.mark.parametrize("order", ["sorted", "shuffled"])
+@pytest.mark.parametrize("n_pairs", [1, 2047, 2048, 2049, None])
+def test_noalloc_chunks_and_full_site_table(order, n_pairs):
+    """1,728 sites, more than one chunk's table of sites holds, on a jittered lattice: a chunk
+    less one pair, one chunk, one more, and every pair inside 5 A; the shuffled list fills the
+    table.  Tolerance as above."""
+    rng = np.random.default_rng(5)
+    g = np.stack(np.meshgrid(*[np.arange(12)] * 3, indexing="ij"), -1).reshape(-1, 3) * 2.5
+    pos, box = g + rng.uniform(-0.4, 0.4, g.shape), np.eye(3) * 30.0
+    d = pos[:, None] - pos[None]
+    d -= np.round(d / 30.0) * 30.0
+    i, j = np.nonzero(np.triu((d ** 2).sum(-1) < 25.0, 1))
+    pairs = np.stack([i, j, np.zeros_like(i)], 1)
+    if order == "shuffled":
+        pairs = pairs[rng.permutation(len(pairs))]
+    pairs = pairs[:n_pairs]
+    prm = rng.uniform(2.0, 4.0, (len(pos), 4))
+    m = np.array([0.0, 0.0, 0.0, 1.0, 1.0, 1.0])
+    ref = _with_context(2, "fp64", pos, box, pairs, m, prm)
+    got = _noalloc(2, "fp64", pos, box, pairs, m, prm)
+    errs = [abs(got[0] - ref[0]) / abs(ref[0])] + [_rel(got[k], ref[k]) for k in (1, 2, 3)]
+    print(f"{order} {len(pairs)} pairs: {errs}", flush=True)
+    assert max(errs) < 1e-12
+
+
 @pytest.mark.parametrize("prec", ["fp64", "mixed"])
 @pytest.mark.parametrize("kind", [1, 2, 3, 4])
 def test_noalloc_equals_context_entry_point_twice(kind, prec):
