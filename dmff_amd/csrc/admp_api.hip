@@ -1191,7 +1191,7 @@ static admp_status admp_get_pairs_impl(admp_ctx* ctx, int32_t frame, int32_t* ou
     HIPCHK(hipStreamSynchronize(ctx->stream));
     *n_out = total;
     if (out && total <= cap)
-        hipLaunchKernelGGL(k_pairs_out, dim3(nblk(N, 256)), dim3(256), 0, ctx->stream, N, ctx->cap, frame, ctx->d_nbr,
+        hipLaunchKernelGGL(k_pairs_out, dim3(nblk(N, 4)), dim3(256), 0, ctx->stream, N, ctx->cap, frame, ctx->d_nbr,
                            ctx->d_ncnt, off, out);
     HIPCHK(hipStreamSynchronize(ctx->stream));
     dfree(ctx, off);

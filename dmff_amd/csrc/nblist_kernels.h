@@ -416,49 +416,76 @@ k_nbr_build(int N, int cap, const double4* __restrict__ pos, const BoxInfo* __re
 }
 
 // reference-format output: rows (i, j, nbond) for j > i, row offsets from an
-// exclusive scan of nhalf (one thread per site)
-__global__ void k_pairs_out(int N, int cap, int f, const int* __restrict__ nbr, const int* __restrict__ ncnt,
-                            const int* __restrict__ off, int* __restrict__ out) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+// exclusive scan of nhalf (one wavefront per site: one thread per site walked a row in
+// dependent steps and wrote single words: 65 us for 29,000 pairs of 648 sites against 3.6)
+__global__ void __launch_bounds__(256)
+k_pairs_out(int N, int cap, int f, const int* __restrict__ nbr, const int* __restrict__ ncnt,
+            const int* __restrict__ off, int* __restrict__ out) {
+    const int i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (i >= N) return;
     const size_t fo = (size_t)f * N;
     const int* row = nbr + (fo + i) * (size_t)cap;
+    const int n = ncnt[fo + i];
     int o = off[i];
-    for (int k = 0; k < ncnt[fo + i]; ++k) {
-        const int w = row[k];
+    for (int k0 = 0; k0 < n; k0 += 64) {
+        const int w = k0 + lane < n ? row[k0 + lane] : 0;
         const int j = w & NB_MASK;
-        if (j > i) {
-            out[o * 3 + 0] = i;
-            out[o * 3 + 1] = j;
-            out[o * 3 + 2] = w >> NB_SHIFT;
-            ++o;
+        const bool keep = k0 + lane < n && j > i;
+        const unsigned long long m = __ballot(keep);
+        if (keep) {
+            int* q = out + (size_t)(o + __popcll(m & ((1ull << lane) - 1ull))) * 3;
+            q[0] = i;
+            q[1] = j;
+            q[2] = w >> NB_SHIFT;
         }
+        o += __popcll(m);
     }
 }
 
-// user pairs (reference format) -> full lists
-template <class I>
-__global__ void k_upairs_count(int64_t np, int N, const I* __restrict__ pairs, int* __restrict__ cnt, int* __restrict__ bad) {
-    const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= np) return;
-    const int64_t i = (int64_t)pairs[r * 3], j = (int64_t)pairs[r * 3 + 1];
-    if (!(i < j)) return;  // padding / i >= j rows vanish (dmff/utils.py:65-84)
-    if (i < 0 || j >= N) { atomicExch(bad, 1); return; }
-    atomicAdd(&cnt[i], 1);
-    atomicAdd(&cnt[j], 1);
+// user pairs (reference format) -> full lists.  A list sorted by its first site gives a
+// wavefront long runs of one i, whose same-address atomics bound these kernels; a run adds
+// once, by its first lane, and its lanes take consecutive places (an unsorted list has runs
+// of one).  Count and fill, 29,000 pairs of 648 sites: 67 and 67 us with an atomic per row,
+// 14 and 14 with one per run.
+__device__ __forceinline__ int run_inc(int* ctr, int i, bool live) {
+    const int lane = threadIdx.x & 63;
+    const int key = live ? i : -1;
+    const int prev = __shfl_up(key, 1, 64);
+    const unsigned long long heads = __ballot(lane == 0 || prev != key);
+    const unsigned long long below = heads & (~0ull >> (63 - lane));         // heads up to this lane
+    const int head = 63 - __clzll((long long)below);
+    const unsigned long long above = head == 63 ? 0 : heads >> (head + 1);   // the next run's head
+    const int len = above ? __ffsll((long long)above) : 64 - head;
+    int base = 0;
+    if (live && lane == head) base = atomicAdd(ctr + i, len);
+    return __shfl(base, head, 64) + (lane - head);
 }
 
 template <class I>
-__global__ void k_upairs_fill(int64_t np, int N, int cap, const I* __restrict__ pairs, int* __restrict__ fill,
-                              int* __restrict__ nbr) {
+__global__ void __launch_bounds__(256)
+k_upairs_count(int64_t np, int N, const I* __restrict__ pairs, int* __restrict__ cnt, int* __restrict__ bad) {
     const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= np) return;
-    const int64_t i = (int64_t)pairs[r * 3], j = (int64_t)pairs[r * 3 + 1];
-    if (!(i < j) || i < 0 || j >= N) return;
+    int64_t i = 0, j = 0;
+    if (r < np) { i = (int64_t)pairs[r * 3]; j = (int64_t)pairs[r * 3 + 1]; }
+    bool live = i < j;  // padding / i >= j rows vanish (dmff/utils.py:65-84)
+    if (live && (i < 0 || j >= N)) { atomicExch(bad, 1); live = false; }
+    run_inc(cnt, (int)i, live);
+    if (live) atomicAdd(&cnt[j], 1);
+}
+
+template <class I>
+__global__ void __launch_bounds__(256)
+k_upairs_fill(int64_t np, int N, int cap, const I* __restrict__ pairs, int* __restrict__ fill,
+              int* __restrict__ nbr) {
+    const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    int64_t i = 0, j = 0;
+    if (r < np) { i = (int64_t)pairs[r * 3]; j = (int64_t)pairs[r * 3 + 1]; }
+    const bool live = i < j && i >= 0 && j < N;
+    const int si = run_inc(fill, (int)i, live);
+    if (!live) return;
     int nb = (int)pairs[r * 3 + 2];
     if (nb < 0) nb = 0;
     if (nb > 7) nb = 7;
-    const int si = atomicAdd(&fill[i], 1);
     const int sj = atomicAdd(&fill[j], 1);
     if (si < cap) nbr[(size_t)i * cap + si] = (int)j | (nb << NB_SHIFT);
     if (sj < cap) nbr[(size_t)j * cap + sj] = (int)i | (nb << NB_SHIFT);

@@ -100,6 +100,7 @@ inline long long __double_as_longlong(double v) { return emu::to_bits(v); }
 inline double __longlong_as_double(long long v) { return emu::from_bits<double>(v); }
 #define __builtin_amdgcn_fence(order, scope) ((void)0)
 inline int __popcll(unsigned long long v) { return __builtin_popcountll(v); }
+inline int __clzll(long long v) { return v ? __builtin_clzll((unsigned long long)v) : 64; }
 inline int __ffsll(long long v) { return __builtin_ffsll(v); }
 template <class T> inline T atomicCAS(T* p, T e, T v) { T o = *p; if (o == e) *p = v; return o; }
 template <class T> inline T atomicAdd(T* p, T v) { T o = *p; *p = o + v; return o; }

@@ -576,6 +576,30 @@ def test_matrix_core_grids(K):
     assert errs.pop("E") < 1e-9 and max(errs.values()) < 1e-7
 
 
+@pytest.mark.parametrize("n_pairs", [1, 63, 64, 65, 257, None])
+def test_pair_rows_in_any_order(n_pairs):
+    """The same pairs sorted, shuffled, and shuffled among padding rows (i >= j, (N, N)): the
+    lists are the same, so the results are equal bit by bit."""
+    from dmff_amd.admp.engine import Engine
+    s, pos, box = _small_waters()
+    rng = np.random.default_rng(3)
+    pairs = np.asarray(reference_pairs(pos, box, 6.0, s.bonded))[:n_pairs]
+    N = len(pos)
+    pad = np.concatenate([pairs[:, [1, 0, 2]], np.full((77, 3), N), np.full((50, 3), 5)])
+    shuffled = pairs[rng.permutation(len(pairs))]
+    mixed = np.concatenate([pairs, pad])
+    mixed = mixed[rng.permutation(len(mixed))]
+    out = []
+    for p in (pairs, shuffled, mixed):
+        eng = Engine(N, 2, False, False, 0.3, (0, 0, 0), 6.0, device=DEV)
+        eng.set_topology(s.axis_types, s.axis_idx, s.bonded)
+        eng.set_pairs(torch.as_tensor(p, device=DEV))
+        E, g, U, info = eng.compute(pos, box, s.pme.Q_local[s.map_atomtype], mScales=s.pme.mScales, want_grad=True)
+        out.append((E.cpu().numpy(), g["pos"].cpu().numpy(), g["Q"].cpu().numpy()))
+    for o in out[1:]:
+        assert all(np.array_equal(a, b) for a, b in zip(o, out[0]))
+
+
 def test_per_frame_pairs_survive_capacity_growth():
     """Pair lists set frame by frame, the second one longer (capacity grows):
     the first frame's list must survive the reallocation (dmff/utils.py:65-84
