@@ -118,7 +118,7 @@ struct admp_ctx {
     double *d_red = nullptr;  // F x 16 scratch reductions
     double *d_red9a = nullptr, *d_red9b = nullptr, *d_red9c = nullptr;
     // solver
-    double *d_b = nullptr, *d_r = nullptr, *d_z = nullptr, *d_p = nullptr, *d_Ap = nullptr, *d_t1 = nullptr,
+    double *d_b = nullptr, *d_r = nullptr, *d_z = nullptr, *d_mrec = nullptr, *d_p = nullptr, *d_Ap = nullptr, *d_t1 = nullptr,
            *d_t2 = nullptr, *d_U = nullptr;
     double *d_dpart = nullptr, *d_dots = nullptr, *d_coef = nullptr, *d_res = nullptr, *d_dU = nullptr;
     PcgState* d_pcg = nullptr;
@@ -753,7 +753,7 @@ extern "C" admp_status admp_ctx_create(const admp_config* cfg, admp_ctx** out) {
     ALLOC(ctx->d_contrib, NF * 12); ALLOC(ctx->d_vir_fr, NF * 9); ALLOC(ctx->d_gQl, NF * 9);
     ALLOC(ctx->d_red, ctx->F * 16);
     ALLOC(ctx->d_red9a, ctx->F * 9); ALLOC(ctx->d_red9b, ctx->F * 9); ALLOC(ctx->d_red9c, ctx->F * 9);
-    ALLOC(ctx->d_b, NF * 3); ALLOC(ctx->d_r, NF * 6); ALLOC(ctx->d_z, NF * 3); ALLOC(ctx->d_p, NF * 3);
+    ALLOC(ctx->d_b, NF * 3); ALLOC(ctx->d_r, NF * 6); ALLOC(ctx->d_z, NF * 3); ALLOC(ctx->d_mrec, NF * MREC); ALLOC(ctx->d_p, NF * 3);
     ALLOC(ctx->d_Ap, NF * 3); ALLOC(ctx->d_t1, NF * 3); ALLOC(ctx->d_t2, NF * 3); ALLOC(ctx->d_U, NF * 3);
     ALLOC(ctx->d_dpart, (size_t)ctx->dots_blocks * ctx->F * 3);
     ALLOC(ctx->d_dots, ctx->F * 3);
@@ -1276,7 +1276,7 @@ template <class R> static const Cplx<R>* twid(const Grid& g, int d) {
 // The real-space product v -> out (FP64 stored coefficients) launched with the
 // plane pass of a solver product (k_plane_matvec)
 struct MatvecJob {
-    const double* v;
+    MatvecRecords src;
     double* out;
 };
 
@@ -1340,8 +1340,8 @@ static admp_status recip_run_mm(admp_ctx* ctx, const Grid& g, int use_dA, const 
             if (mv) {
                 const int npb = xcd_blocks(H * F), nbf = (int)nblk((size_t)N * TPA, th);
                 hipLaunchKernelGGL(k_plane_mm_matvec<NT>, dim3(npb + xcd_blocks(nbf * F)), dim3(th), sm, st, K0, K1, K2, tx,
-                                   ty, hg, q, F, npb, N, nbf, ctx->cap, ctx->d_pos, ctx->d_nbr, ctx->d_ncnt,
-                                   reinterpret_cast<const double*>(ctx->d_pcoef), mv->v, mv->out, skip);
+                                   ty, hg, q, F, npb, N, nbf, ctx->cap, ctx->d_nbr, ctx->d_ncnt,
+                                   reinterpret_cast<const double*>(ctx->d_pcoef), mv->src, mv->out, skip);
             } else if (in == IN_TABLE) {
                 hipLaunchKernelGGL((k_plane_mm<NT, IN_TABLE>), dim3(H, F), dim3(th), sm, st, K0, K1, K2, tx, ty, hg, q, skip);
             } else if (in == IN_TABLE_ACC) {
@@ -1555,8 +1555,8 @@ static admp_status recip_run(admp_ctx* ctx, const Grid& g, int use_dA, const dou
             const int nbf = (int)nblk((size_t)N * TPA, PLANE_THREADS);
             hipLaunchKernelGGL((k_plane_matvec<R>), dim3(npb + xcd_blocks(nbf * F)), dim3(PLANE_THREADS), sm, st, K0, K1,
                                K2, g.plan[0], g.plan[1], twid<R>(g, 0), twid<R>(g, 1), hg, ctx->d_box, g.bmod[0], g.bmod[1],
-                               g.bmod[2], kappa, kind, pref, tab, F, npb, N, nbf, ctx->cap, ctx->d_pos, ctx->d_nbr,
-                               ctx->d_ncnt, reinterpret_cast<const double*>(ctx->d_pcoef), mv->v, mv->out, skip);
+                               g.bmod[2], kappa, kind, pref, tab, F, npb, N, nbf, ctx->cap, ctx->d_nbr,
+                               ctx->d_ncnt, reinterpret_cast<const double*>(ctx->d_pcoef), mv->src, mv->out, skip);
         } else
             hipLaunchKernelGGL((k_fxy_plane<R, false>), dim3(H, F), dim3(PLANE_THREADS), sm, st, K0, K1, K2, g.plan[0], g.plan[1],
                                twid<R>(g, 0), twid<R>(g, 1), hg, ctx->d_box, g.bmod[0], g.bmod[1], g.bmod[2], kappa,
@@ -1618,9 +1618,9 @@ static admp_status matvec(admp_ctx* ctx, const double* v, double* out, const dou
     }
     { ProfScope ps_(ctx, 2);
     const int nbf = (int)nblk((size_t)N * TPA, PAIR_BLOCK);
-    hipLaunchKernelGGL((k_real_matvec<RC, R>), dim3(xcd_blocks(nbf * F)), dim3(PAIR_BLOCK), 0, st, N, nbf, F,
-                       ctx->cap, ctx->d_pos, ctx->d_box, ctx->d_nbr, ctx->d_ncnt,
-                       reinterpret_cast<const RC*>(ctx->d_pcoef), vR, ctx->d_t1, (const PcgState*)nullptr); }
+    hipLaunchKernelGGL((k_real_matvec<RC, R, MatvecArrays<R>>), dim3(xcd_blocks(nbf * F)), dim3(PAIR_BLOCK), 0, st, N, nbf,
+                       F, ctx->cap, ctx->d_box, ctx->d_nbr, ctx->d_ncnt, reinterpret_cast<const RC*>(ctx->d_pcoef),
+                       (MatvecArrays<R>{ctx->d_pos, vR}), ctx->d_t1, (const PcgState*)nullptr); }
     double* rec = nullptr;
     if (ctx->cfg.lpme) {
         admp_status s = recip_run<R>(ctx, ctx->eg, 0, nullptr, v, 2, 1, 0, DIELECTRIC, ctx->cfg.kappa, 1, ctx->d_t2,
@@ -1668,26 +1668,29 @@ template <class RC, class R>
 static admp_status pcg_apply(admp_ctx* ctx, const double* pol, double f1, int cur, double tol) {
     const int N = ctx->N, F = ctx->F;
     hipStream_t st = ctx->stream;
-    // real-space products in FP64 whenever the stored coefficients are FP64 (the
-    // near-field coupling sets the conditioning); R only for the reciprocal chain
-    using RR = typename std::conditional<sizeof(RC) == 8, double, R>::type;
-    const RR* vR = sizeof(RR) == 8 ? reinterpret_cast<const RR*>(ctx->d_z) : reinterpret_cast<const RR*>(ctx->d_vR);
+    // real-space products in FP64, as the stored coefficients are (the near-field
+    // coupling sets the conditioning); R only for the reciprocal chain
+    static_assert(sizeof(RC) == 8, "the records hold FP64");
+    const MatvecRecords rec{reinterpret_cast<const double2*>(ctx->d_mrec)};
     const bool fused = ctx->cfg.lpme && !small_grid(ctx->eg);
     // With few frames the plane pass fills only K2/2+1 workgroups per frame: the
     // real-space product then runs inside that launch (k_plane_matvec) instead of
-    // on the side stream, which saves the fork and the join of every iteration.
-    const int H = ctx->eg.K[2] / 2 + 1;
+    // on the side stream, which saves the fork and the join of every iteration, as
+    // long as the CUs without a plane hold its lanes at once (98,304 sites beside 41
+    // planes of 80 x 80 are 3.6 rounds of them: 490 us per iteration in one launch
+    // against 460 on the side stream).
+    const int np = (ctx->eg.K[2] / 2 + 1) * F;
     const bool plane = sizeof(R) == 8 && ctx->eg.mm ? ctx->eg.mm_plane : ctx->eg.plane[sizeof(R) == 8 ? 1 : 0];
-    const bool with_plane = fused && sizeof(RC) == 8 && plane && H * F <= 128;
+    const bool with_plane = fused && plane && np <= 128 && (long)N * F * TPA <= 2048L * (256 - np);
     if (!with_plane) {
         // the real-space product runs on the side stream, beside the reciprocal chain
         HIPCHK(hipEventRecord(ctx->ev_fork, st));
         HIPCHK(hipStreamWaitEvent(ctx->side, ctx->ev_fork, 0));
         { ProfScope ps_(ctx, 2, ctx->side);
         const int nbf = (int)nblk((size_t)N * TPA, PAIR_BLOCK);
-        hipLaunchKernelGGL((k_real_matvec<RC, RR>), dim3(xcd_blocks(nbf * F)), dim3(PAIR_BLOCK), 0, ctx->side, N, nbf,
-                           F, ctx->cap, ctx->d_pos, ctx->d_box, ctx->d_nbr, ctx->d_ncnt,
-                           reinterpret_cast<const RC*>(ctx->d_pcoef), vR, ctx->d_t1, ctx->d_pcg); }
+        hipLaunchKernelGGL((k_real_matvec<RC, double, MatvecRecords>), dim3(xcd_blocks(nbf * F)), dim3(PAIR_BLOCK), 0,
+                           ctx->side, N, nbf, F, ctx->cap, ctx->d_box, ctx->d_nbr, ctx->d_ncnt,
+                           reinterpret_cast<const RC*>(ctx->d_pcoef), rec, ctx->d_t1, ctx->d_pcg); }
         HIPCHK(hipEventRecord(ctx->ev_join, ctx->side));
     }
     // the product's first kernel tests the residual the next update would test
@@ -1695,7 +1698,7 @@ static admp_status pcg_apply(admp_ctx* ctx, const double* pol, double f1, int cu
     admp_status s = ADMP_OK;
     if (with_plane) {
         const CgEpi epi{ctx->d_t1, pol, f1, cg_parts(ctx)};
-        const MatvecJob mv{ctx->d_z, ctx->d_t1};
+        const MatvecJob mv{rec, ctx->d_t1};
         s = recip_run<R>(ctx, ctx->eg, 0, nullptr, ctx->d_z, 2, 1, 0, DIELECTRIC, ctx->cfg.kappa, 2, ctx->d_Ap,
                          nullptr, nullptr, nullptr, false, ctx->d_swfrac, ctx->d_sfq, ctx->d_pcg, &epi, nullptr, &mv);
         ctx->cg_nwu = gather_parts<R>(ctx);
@@ -1731,7 +1734,7 @@ template <class R>
 static void launch_update(admp_ctx* ctx, int cur, double* x, double tol, const double* pol) {
     hipLaunchKernelGGL(k_cg_update<R>, dim3(ctx->pcg_nb, ctx->F), dim3(PCG_BLOCK), 0, ctx->stream, ctx->N,
                        ctx->cg_nwu, cur, tol, ctx->d_box, pol, x, ctx->d_r, ctx->d_z, ctx->d_p, ctx->d_s, ctx->d_Ap,
-                       sizeof(R) == 8 ? nullptr : reinterpret_cast<R*>(ctx->d_vR),
+                       ctx->d_mrec,
                        ctx->cfg.lpme ? reinterpret_cast<R*>(ctx->d_sfq) : nullptr, pc_j(ctx), ctx->d_pcd,
                        cg_parts(ctx), ctx->d_pcg);
 }
@@ -1754,13 +1757,13 @@ static admp_status pcg_restart(admp_ctx* ctx, const double* rhs, const double* x
     const double* wd = ctx->cfg.lpme ? ctx->d_wd : nullptr;
     if (dbl)
         hipLaunchKernelGGL(k_cg_start<double>, dim3(ctx->pcg_nb, F), dim3(PCG_BLOCK), 0, st, N, ctx->d_box, wd, pol,
-                           rhs, Ax, ctx->d_r, ctx->d_z, (double*)nullptr,
+                           rhs, Ax, ctx->d_r, ctx->d_z, ctx->d_pos, ctx->d_mrec,
                            reinterpret_cast<double*>(ctx->d_swfrac),
                            ctx->cfg.lpme ? reinterpret_cast<double*>(ctx->d_sfq) : nullptr, pc_j(ctx), ctx->d_pcd,
                            cg_parts(ctx), xz);
     else
         hipLaunchKernelGGL(k_cg_start<float>, dim3(ctx->pcg_nb, F), dim3(PCG_BLOCK), 0, st, N, ctx->d_box, wd, pol,
-                           rhs, Ax, ctx->d_r, ctx->d_z, reinterpret_cast<float*>(ctx->d_vR),
+                           rhs, Ax, ctx->d_r, ctx->d_z, ctx->d_pos, ctx->d_mrec,
                            reinterpret_cast<float*>(ctx->d_swfrac),
                            ctx->cfg.lpme ? reinterpret_cast<float*>(ctx->d_sfq) : nullptr, pc_j(ctx), ctx->d_pcd,
                            cg_parts(ctx), xz);

@@ -1003,18 +1003,51 @@ k_pc_clusters(int N, int cap, int maxm, const double4* __restrict__ pos, const B
 // holds the positions and v of few frames).  nbf: atom blocks per frame.
 // item: (frame, atom block of BS threads) pair, numbered frame-major; nbf atom
 // blocks per frame
-template <bool ORTHO, class RC, class R>
-__device__ __forceinline__ void real_matvec_pairs(int sub, int cnt, const BoxInfo& bx, const double4& pi_,
-                                                  const double4* __restrict__ posf, const R* __restrict__ vf,
+// The neighbours' positions and vectors: from their own arrays (any v), or from the solver's
+// records of six doubles, position and z, which k_cg_start and k_cg_update keep.  The loop is
+// bound by these random loads: a record is three aligned 16-byte loads where the two arrays
+// take five (64 frames of 12,288 sites with 215 neighbours each: 1185 -> 1065 us beside the
+// spread; 98,304 sites with 420: 298 -> 257 us).
+template <class R> struct MatvecArrays {
+    const double4* __restrict__ pos;
+    const R* __restrict__ v;
+    __device__ __forceinline__ void frame(size_t fo) { pos += fo; v += fo * 3; }
+    __device__ __forceinline__ double4 at(int j) const { return pos[j]; }
+    __device__ __forceinline__ void load(int j, double& x, double& y, double& z, R& vx, R& vy, R& vz) const {
+        const double4 p = pos[j];
+        const R* w = v + 3 * j;
+        x = p.x; y = p.y; z = p.z;
+        vx = w[0]; vy = w[1]; vz = w[2];
+    }
+};
+constexpr int MREC = 6;
+struct MatvecRecords {
+    const double2* __restrict__ rec;
+    __device__ __forceinline__ void frame(size_t fo) { rec += fo * (MREC / 2); }
+    __device__ __forceinline__ double4 at(int j) const {
+        const double2 a = rec[3 * j], b = rec[3 * j + 1];
+        return make_double4(a.x, a.y, b.x, 0.0);
+    }
+    __device__ __forceinline__ void load(int j, double& x, double& y, double& z, double& vx, double& vy, double& vz) const {
+        const double2 a = rec[3 * j], b = rec[3 * j + 1], c = rec[3 * j + 2];
+        x = a.x; y = a.y; z = b.x;
+        vx = b.y; vy = c.x; vz = c.y;
+    }
+};
+
+template <bool ORTHO, class RC, class R, class SRC>
+__device__ __forceinline__ void real_matvec_pairs(int sub, int cnt, const BoxInfo& bx, const double4& pi_, const SRC& src,
                                                   const int* __restrict__ nl, const RC* __restrict__ pc, double& ox,
                                                   double& oy, double& oz) {
     // one neighbour per trip: the loop is bound by the random position and
     // direction loads, and the fewer registers of a plain loop beat two or four
-    // neighbours per trip (64-frame batch: 2.3 % and 5 % faster).  posf and vf
-    // are the frame's bases, so the per-neighbour offsets are 32-bit.
+    // neighbours per trip (64-frame batch: 2.3 % and 5 % faster).  src is the
+    // frame's, so the per-neighbour offsets are 32-bit.
     auto term = [&](int j, RC c1r, RC c2r) {
-        const double4 pj = posf[j];
-        double dx = pi_.x - pj.x, dy = pi_.y - pj.y, dz = pi_.z - pj.z;
+        double jx, jy, jz;
+        R vx, vy, vz;
+        src.load(j, jx, jy, jz, vx, vy, vz);
+        double dx = pi_.x - jx, dy = pi_.y - jy, dz = pi_.z - jz;
         if constexpr (ORTHO) {
             // the general minimum image of pbc_shift with zero off-diagonal
             // terms (which add exact zeros there): the same value
@@ -1027,8 +1060,6 @@ __device__ __forceinline__ void real_matvec_pairs(int sub, int cnt, const BoxInf
             pbc_shift(bx, dx, dy, dz, n0, n1, n2);
         }
         const R ex = (R)dx, ey = (R)dy, ez = (R)dz;
-        const R* vj = vf + 3 * j;
-        const R vx = vj[0], vy = vj[1], vz = vj[2];
         const R c1 = (R)c1r, c2 = (R)c2r;
         const R p = c2 * (ex * vx + ey * vy + ez * vz);
         ox += (double)(c1 * vx + p * ex);
@@ -1038,12 +1069,11 @@ __device__ __forceinline__ void real_matvec_pairs(int sub, int cnt, const BoxInf
     for (int k = sub; k < cnt; k += TPA) term(nl[k] & NB_MASK, pc[2 * k], pc[2 * k + 1]);
 }
 
-template <class RC, class R>
-__device__ __forceinline__ void real_matvec_body(int BS, int item, int N, int nbf, int cap, const double4* __restrict__ pos,
+template <class RC, class R, class SRC>
+__device__ __forceinline__ void real_matvec_body(int BS, int item, int N, int nbf, int cap,
                                                  const BoxInfo* __restrict__ boxes, const int* __restrict__ nbr,
-                                                 const int* __restrict__ ncnt, const RC* __restrict__ pcoef,
-                                                 const R* __restrict__ v, double* __restrict__ out,
-                                                 const PcgState* __restrict__ skip) {
+                                                 const int* __restrict__ ncnt, const RC* __restrict__ pcoef, SRC src,
+                                                 double* __restrict__ out, const PcgState* __restrict__ skip) {
     const int f = item / nbf, bxi = item - f * nbf;
     if (skip && skip[f].done) return;  // frame already converged
     const int gt = bxi * BS + threadIdx.x;
@@ -1052,17 +1082,16 @@ __device__ __forceinline__ void real_matvec_body(int BS, int item, int N, int nb
     const int ii = active ? i : 0;
     const BoxInfo& bx = boxes[f];
     const size_t fo = (size_t)f * N;
-    const double4* posf = pos + fo;
-    const R* vf = v + fo * 3;
-    const double4 pi_ = posf[ii];
+    src.frame(fo);
+    const double4 pi_ = src.at(ii);
     double ox = 0, oy = 0, oz = 0;
     const int cnt = active ? ncnt[fo + ii] : 0;
     const int* nl = nbr + (fo + ii) * (size_t)cap;
     const RC* pc = pcoef + (fo + ii) * (size_t)cap * 2;
     if (bx.ortho)
-        real_matvec_pairs<true>(sub, cnt, bx, pi_, posf, vf, nl, pc, ox, oy, oz);
+        real_matvec_pairs<true, RC, R>(sub, cnt, bx, pi_, src, nl, pc, ox, oy, oz);
     else
-        real_matvec_pairs<false>(sub, cnt, bx, pi_, posf, vf, nl, pc, ox, oy, oz);
+        real_matvec_pairs<false, RC, R>(sub, cnt, bx, pi_, src, nl, pc, ox, oy, oz);
     ox = group_sum(ox, TPA); oy = group_sum(oy, TPA); oz = group_sum(oz, TPA);
     if (active && sub == 0) {
         const size_t a = fo + i;
@@ -1070,14 +1099,14 @@ __device__ __forceinline__ void real_matvec_body(int BS, int item, int N, int nb
     }
 }
 
-template <class RC, class R>
+template <class RC, class R, class SRC>
 __global__ void __launch_bounds__(PAIR_BLOCK)
-k_real_matvec(int N, int nbf, int F, int cap, const double4* __restrict__ pos, const BoxInfo* __restrict__ boxes,
-              const int* __restrict__ nbr, const int* __restrict__ ncnt, const RC* __restrict__ pcoef,
-              const R* __restrict__ v, double* __restrict__ out, const PcgState* __restrict__ skip) {
+k_real_matvec(int N, int nbf, int F, int cap, const BoxInfo* __restrict__ boxes, const int* __restrict__ nbr,
+              const int* __restrict__ ncnt, const RC* __restrict__ pcoef, SRC src, double* __restrict__ out,
+              const PcgState* __restrict__ skip) {
     const int item = xcd_item(blockIdx.x, nbf * F);
     if (item >= nbf * F) return;
-    real_matvec_body<RC, R>(PAIR_BLOCK, item, N, nbf, cap, pos, boxes, nbr, ncnt, pcoef, v, out, skip);
+    real_matvec_body<RC, R>(PAIR_BLOCK, item, N, nbf, cap, boxes, nbr, ncnt, pcoef, src, out, skip);
 }
 
 }  // namespace admp

@@ -1360,8 +1360,8 @@ k_plane_matvec(int K0, int K1, int K2, FFTPlan plan0, FFTPlan plan1, const Cplx<
                const Cplx<R>* __restrict__ tw1g, Cplx<R>* __restrict__ hgrid, const BoxInfo* __restrict__ boxes,
                const double* __restrict__ bmod0, const double* __restrict__ bmod1, const double* __restrict__ bmod2,
                double kappa, int kind, double pref, const double* __restrict__ tab, int F, int nplane_blocks,
-               int N, int nbf, int cap, const double4* __restrict__ pos, const int* __restrict__ nbr,
-               const int* __restrict__ ncnt, const double* __restrict__ pcoef, const double* __restrict__ v,
+               int N, int nbf, int cap, const int* __restrict__ nbr,
+               const int* __restrict__ ncnt, const double* __restrict__ pcoef, MatvecRecords src,
                double* __restrict__ out, const PcgState* __restrict__ skip) {
     const int H = K2 / 2 + 1;
     const int b = blockIdx.x;
@@ -1375,7 +1375,7 @@ k_plane_matvec(int K0, int K1, int K2, FFTPlan plan0, FFTPlan plan1, const Cplx<
     }
     const int item = xcd_item(b - nplane_blocks, nbf * F);
     if (item >= nbf * F) return;
-    real_matvec_body<double, double>(PLANE_THREADS, item, N, nbf, cap, pos, boxes, nbr, ncnt, pcoef, v, out, skip);
+    real_matvec_body<double, double>(PLANE_THREADS, item, N, nbf, cap, boxes, nbr, ncnt, pcoef, src, out, skip);
 }
 
 }  // namespace admp

@@ -631,8 +631,8 @@ template <int NT>
 __global__ void __launch_bounds__(MM_PT(NT))
 k_plane_mm_matvec(int K0, int K1, int K2, const Cplx<double>* __restrict__ twx, const Cplx<double>* __restrict__ twy,
                   Cplx<double>* __restrict__ hgrid, InflArgs q, int F, int nplane_blocks, int N, int nbf, int cap,
-                  const double4* __restrict__ pos, const int* __restrict__ nbr, const int* __restrict__ ncnt,
-                  const double* __restrict__ pcoef, const double* __restrict__ v, double* __restrict__ out,
+                  const int* __restrict__ nbr, const int* __restrict__ ncnt,
+                  const double* __restrict__ pcoef, MatvecRecords src, double* __restrict__ out,
                   const PcgState* __restrict__ skip) {
     const int H = K2 / 2 + 1;
     const int b = blockIdx.x;
@@ -644,7 +644,7 @@ k_plane_mm_matvec(int K0, int K1, int K2, const Cplx<double>* __restrict__ twx, 
     }
     const int item = xcd_item(b - nplane_blocks, nbf * F);
     if (item >= nbf * F) return;
-    real_matvec_body<double, double>(blockDim.x, item, N, nbf, cap, pos, q.boxes, nbr, ncnt, pcoef, v, out, skip);
+    real_matvec_body<double, double>(blockDim.x, item, N, nbf, cap, q.boxes, nbr, ncnt, pcoef, src, out, skip);
 }
 
 // Planes too large for LDS: y lines and x lines in passes of their own, 32 lines per

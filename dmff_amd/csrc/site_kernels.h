@@ -823,12 +823,11 @@ __device__ inline double block_red(double v, double* sh) {
 
 __device__ inline double inv_diag(double pol) { return (pol < 1e-8 ? 1e-8 : pol) / DIELECTRIC; }
 
-// the product inputs derived from z: its R copy for the pair kernel and the
+// the product inputs derived from z: its place in the pair kernel's records and the
 // fractional dipoles A^T z (slots 1..3 of the 10-wide fractional multipoles)
 template <class R>
-__device__ inline void cg_derived(const BoxInfo* __restrict__ boxes, int f, size_t a, const double* u, R* zR, R* fq) {
-    if (zR)
-        for (int k = 0; k < 3; ++k) zR[a * 3 + k] = (R)u[k];
+__device__ inline void cg_derived(const BoxInfo* __restrict__ boxes, int f, size_t a, const double* u, double* rec, R* fq) {
+    for (int k = 0; k < 3; ++k) rec[a * MREC + 3 + k] = u[k];
     if (!fq) return;
     const double* A = boxes[f].A;
     R* o = fq + a * 10;
@@ -866,7 +865,8 @@ __global__ void __launch_bounds__(PCG_BLOCK) k_cg_start(int N, const BoxInfo* __
                                                         const double* __restrict__ wd, const double* __restrict__ pol,
                                                         const double* __restrict__ b, const double* __restrict__ Ax,
                                                         double* __restrict__ r, double* __restrict__ z,
-                                                        R* __restrict__ zR, R* __restrict__ wfrac, R* __restrict__ fq,
+                                                        const double4* __restrict__ pos, double* __restrict__ rec,
+                                                        R* __restrict__ wfrac, R* __restrict__ fq,
                                                         const int* __restrict__ pcj, const double* __restrict__ pcd,
                                                         CgParts parts, double* __restrict__ xzero) {
     __shared__ double sh[16];
@@ -902,7 +902,9 @@ __global__ void __launch_bounds__(PCG_BLOCK) k_cg_start(int N, const BoxInfo* __
             o[0] = 0;
             for (int k = 4; k < 10; ++k) o[k] = 0;
         }
-        cg_derived<R>(boxes, f, a, u, zR, fq);
+        const double4 p = pos[a];
+        rec[a * MREC] = p.x; rec[a * MREC + 1] = p.y; rec[a * MREC + 2] = p.z;
+        cg_derived<R>(boxes, f, a, u, rec, fq);
     }
     rz = block_red<false>(rz, sh);
     mx = block_red<true>(mx, sh);
@@ -967,7 +969,7 @@ __global__ void __launch_bounds__(PCG_BLOCK) k_cg_update(int N, int nwu, int cur
                                                          const double* __restrict__ pol, double* __restrict__ x,
                                                          double* __restrict__ r, double* __restrict__ z,
                                                          double* __restrict__ p, double* __restrict__ s,
-                                                         const double* __restrict__ w, R* __restrict__ zR,
+                                                         const double* __restrict__ w, double* __restrict__ rec,
                                                          R* __restrict__ fq, const int* __restrict__ pcj,
                                                          const double* __restrict__ pcd, CgParts parts,
                                                          PcgState* __restrict__ st) {
@@ -1055,7 +1057,7 @@ __global__ void __launch_bounds__(PCG_BLOCK) k_cg_update(int N, int nwu, int cur
             z[a * 3 + k] = u[k];
             lrz += rv[k] * u[k];
         }
-        cg_derived<R>(boxes, f, a, u, zR, fq);
+        cg_derived<R>(boxes, f, a, u, rec, fq);
     }
     lrz = block_red<false>(lrz, sh);
     lmx = block_red<true>(lmx, sh);
