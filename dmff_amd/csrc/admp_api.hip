@@ -98,6 +98,8 @@ struct admp_ctx {
     int2* d_blist = nullptr;                        // per-brick candidate lists
     double* d_infl = nullptr;                       // tabulated electrostatic influence function (eg)
     int infl_pm = 0;                                // its layout: plane-major (1) or line-major (0)
+    // a solve with FP32 products is running: its FP64 passes take the radix path (use_mm)
+    bool radix64 = false;
     bool plane_lds_ok = false;                      // plane kernels may use PLANE_LDS_MAX bytes of LDS
     long blist_cap = 0;
     int* d_scan_tmp = nullptr;  // tile totals of scan_rows
@@ -431,6 +433,14 @@ static bool mm_kernels_ready() {
     }();
     return ok;
 }
+
+// The FP64 passes run on the matrix cores, except in a solve with FP32 products (the Jacobi
+// sweeps of a mixed context, CG with fp32_products).  There the right-hand side's last bit
+// decides how the products round: with the matrix-core passes, which agree with the radix
+// ones to 1e-15, the dipoles of an 882-site sheared box come out 3e-8 apart after ten
+// sweeps, so such a solve keeps the passes, and the results, that it has had.  They are a
+// small part of it: the sweeps run the FP32 radix passes either way.
+static bool use_mm(const admp_ctx* ctx, const Grid& g) { return g.mm && !ctx->radix64; }
 
 // ADMP_SPREAD=list|col|cw forces a spread of the radix path (measurements)
 static int spread_forced() {
@@ -1231,7 +1241,7 @@ static admp_status recip_positions(admp_ctx* ctx, const Grid& g, int use_dA) {
         if (&g == &ctx->eg && ctx->d_infl && !use_dA) {
             const size_t nt = (size_t)g.K[0] * g.K[1] * (g.K[2] / 2 + 1);
             // laid out for the FP64 solver products' FFT path
-            ctx->infl_pm = g.mm || g.plane[1] ? 1 : 0;
+            ctx->infl_pm = use_mm(ctx, g) || g.plane[1] ? 1 : 0;
             hipLaunchKernelGGL(k_infl_table, dim3(nblk(nt, 256), F), dim3(256), 0, st, g.K[0], g.K[1], g.K[2],
                                ctx->d_box, g.bmod[0], g.bmod[1], g.bmod[2], ctx->cfg.kappa, DIELECTRIC, ctx->infl_pm,
                                ctx->d_infl);
@@ -1408,7 +1418,7 @@ static admp_status recip_run_mm(admp_ctx* ctx, const Grid& g, int use_dA, const 
 // z.w partials the CG epilogue of the gather leaves per frame
 template <class R> static int gather_parts(const admp_ctx* ctx) {
     const Grid& g = ctx->eg;
-    return sizeof(R) == 8 && g.mm ? ((g.K[0] + MM_TX - 1) / MM_TX) * ((g.K[1] + MM_TY - 1) / MM_TY) : gather_blocks(ctx->N);
+    return sizeof(R) == 8 && use_mm(ctx, g) ? ((g.K[0] + MM_TX - 1) / MM_TX) * ((g.K[1] + MM_TY - 1) / MM_TY) : gather_blocks(ctx->N);
 }
 
 // Spread the sources (Qc, U, qmode), transform, apply the influence function,
@@ -1434,7 +1444,7 @@ static admp_status recip_run(admp_ctx* ctx, const Grid& g, int use_dA, const dou
                            ctx->d_wd, wfrac, fq);
     }
     if constexpr (sizeof(R) == 8) {
-        if (g.mm)
+        if (use_mm(ctx, g))
             return recip_run_mm(ctx, g, use_dA, Qc, U, qmode, lmax_eff, kind, pref, kappa, gather_mode, out3, gq, gpos,
                                 vir, want_energy, wfrac, fq, skip, epi, before_gather, mv);
     }
@@ -1680,7 +1690,7 @@ static admp_status pcg_apply(admp_ctx* ctx, const double* pol, double f1, int cu
     // planes of 80 x 80 are 3.6 rounds of them: 490 us per iteration in one launch
     // against 460 on the side stream).
     const int np = (ctx->eg.K[2] / 2 + 1) * F;
-    const bool plane = sizeof(R) == 8 && ctx->eg.mm ? ctx->eg.mm_plane : ctx->eg.plane[sizeof(R) == 8 ? 1 : 0];
+    const bool plane = sizeof(R) == 8 && use_mm(ctx, ctx->eg) ? ctx->eg.mm_plane : ctx->eg.plane[sizeof(R) == 8 ? 1 : 0];
     const bool with_plane = fused && plane && np <= 128 && (long)N * F * TPA <= 2048L * (256 - np);
     if (!with_plane) {
         // the real-space product runs on the side stream, beside the reciprocal chain
@@ -1830,7 +1840,7 @@ static admp_status pcg(admp_ctx* ctx, const double* rhs, double* x, const double
             return ADMP_OK;
         };
         if (!ctx->use_graphs) return iterate();
-        const int type = (sizeof(RC) == 8 ? 1 : 0) + (use_dbl ? 2 : 0);
+        const int type = (sizeof(RC) == 8 ? 1 : 0) + (use_dbl ? 2 : 0) + (ctx->radix64 ? 4 : 0);
         admp_ctx::ChunkGraph* cg = nullptr;
         auto same = [&](const admp_ctx::ChunkGraph& g) {
             return g.type == type && g.nrun == nrun && g.par == par && g.rhs == rhs && g.x == x && g.tol == tol &&
@@ -2094,6 +2104,11 @@ static admp_status solve(admp_ctx* ctx, const double* pol, const double* thole, 
     const bool warm = o && o->warm_start && U_in;
     const bool fp32 = mixed && o && o->fp32_products;
     const bool started = kind == ADMP_SOLVER_PCG && !fp32 && !warm;   // see below
+    struct Radix64 {
+        admp_ctx* ctx;
+        ~Radix64() { ctx->radix64 = false; }
+    } radix64{ctx};
+    ctx->radix64 = mixed && (kind != ADMP_SOLVER_PCG || fp32);
     if (warm)
         HIPCHK(hipMemcpyAsync(U, U_in, NF * 3 * sizeof(double), hipMemcpyDeviceToDevice, st));
     else if (!started)
@@ -2120,7 +2135,7 @@ static admp_status solve(admp_ctx* ctx, const double* pol, const double* thole, 
         // state its capture left): later launches and captures must not sort again
         if (c.lpme) {
             ctx->prepped = &ctx->eg;
-            (ctx->eg.mm ? ctx->tiles_ok : ctx->bricks_ok) = true;
+            (use_mm(ctx, ctx->eg) ? ctx->tiles_ok : ctx->bricks_ok) = true;
         }
     } else {
         if ((s = launch_frames_fwd(ctx)) != ADMP_OK) return s;
