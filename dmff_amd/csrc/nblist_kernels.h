@@ -367,8 +367,30 @@ k_nbr_build(int N, int cap, const double4* __restrict__ pos, const BoxInfo* __re
     if (lane < ncand) {
         const int a2 = lane % nl[2], a1 = (lane / nl[2]) % nl[1], a0 = lane / (nl[2] * nl[1]);
         const int cid = (lst[0][a0] * cg.nc[1] + lst[1][a1]) * cg.nc[2] + lst[2][a2];
-        mylo = cs[cid];
-        myhi = cs[cid + 1];
+        // A cell further than rc from the site has no neighbours: 17 of 27 cells remain on
+        // average where cells are little wider than rc (98,304 sites at rc 10: 840 -> 662 us; 64
+        // frames of 12,288 at rc 8: 3.49 -> 3.11 ms; one such frame, latency bound: 67 -> 65 us).
+        // The distance to the cell's slab along each axis is a lower bound; in an orthogonal
+        // box the three add up.  (The far side of a cell, reached the other way round, is at
+        // least a cell's width off.)  1e-6 A covers the rounding of cell membership.
+        const int at[3] = {lst[0][a0], lst[1][a1], lst[2][a2]};
+        double sum = 0, most = 0;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            const double* Bi = bm.Binv + d;
+            double sd = pi_.x * Bi[0] + pi_.y * Bi[3] + pi_.z * Bi[6];
+            sd = (sd - floor(sd)) * cg.nc[d] - cc[d];                       // place in the own cell, 0..1
+            const int n = cg.nc[d], off = (at[d] - cc[d] + n) % n;
+            const double up = off == 1 ? 1.0 - sd : 1e30, down = off == n - 1 ? sd : 1e30;
+            const double w = 1.0 / (n * sqrt(Bi[0] * Bi[0] + Bi[3] * Bi[3] + Bi[6] * Bi[6]));   // slab width
+            const double g = off == 0 ? 0.0 : fmax(0.0, fmin(up, down) * w - 1e-6);
+            sum += g * g;
+            most = fmax(most, g * g);
+        }
+        if ((ortho ? sum : most) < rc2) {
+            mylo = cs[cid];
+            myhi = cs[cid + 1];
+        }
     }
     for (int q = 0; q < ncand; ++q) {
         const int lo = __shfl(mylo, q, 64), hi = __shfl(myhi, q, 64);

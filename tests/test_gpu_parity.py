@@ -230,6 +230,34 @@ def test_neighbor_list_bit_exact():
         assert len(a) > 0 and a.shape == b.shape and np.array_equal(a, b), name
 
 
+@pytest.mark.parametrize("cells", [(2, 3, 4), (3, 3, 3), (4, 5, 3), (6, 2, 1)])
+@pytest.mark.parametrize("tilt", [0.0, 0.35])
+def test_neighbor_list_skipped_cells(cells, tilt):
+    """Cells barely wider than the cutoff, where most corner cells are out of a site's reach,
+    in orthogonal and sheared boxes, sites outside the cell of the box among them: the pairs of
+    all sites against all sites under the same minimum image."""
+    from dmff_amd.admp.engine import Engine
+    rng = np.random.default_rng(sum(cells))
+    rc, n = 4.0, 500
+    box = np.diag([c * rc * 1.004 for c in cells])
+    box[1, 0], box[2, 1] = tilt * box[0, 0], -tilt * box[1, 1]
+    frac = rng.uniform(-1.0, 2.0, (n, 3))
+    frac[:60] = np.round(frac[:60] * cells) / cells      # on the cells' faces
+    pos = frac @ box
+    eng = Engine(n, 0, False, False, 0.0, (0, 0, 0), rc, device=DEV)
+    eng.set_topology(None, None, {})
+    # slabs narrower than rc (sheared boxes) make fewer cells; the list is the same
+    eng.build_neighbors(pos, box)
+    got = eng.get_pairs(0).cpu().numpy().astype(np.int64)[:, :2]
+    s = (pos[:, None] - pos[None]) @ np.linalg.inv(box)
+    r2 = (((s - np.floor(s + 0.5)) @ box) ** 2).sum(-1)
+    sure = np.abs(r2 - rc * rc) > 1e-9
+    ref = np.triu(r2 < rc * rc, 1)
+    hit = np.zeros((n, n), bool)
+    hit[got[:, 0], got[:, 1]] = True
+    assert len(got) == hit.sum() and np.array_equal(hit[sure], ref[sure])
+
+
 def test_mixed_precision_error_bounds():
     s, pos, box = _small_waters()
     pairs = reference_pairs(pos, box, 6.0, s.bonded)
