@@ -593,8 +593,8 @@ def pair_kernel_valu(us_mixed):
     return out or None
 
 
-DOMINANT_KERNEL_SOURCE = ("k_plane_matvec<double>: 19.6 % of the kernel time of the timed evaluations, ahead of "
-                          "k_spread_cw<double, 1, 48> (16.0 %), profiles/admp_12288_kernel_stats.md")
+DOMINANT_KERNEL_SOURCE = ("k_plane_mm_matvec<2>: 23.3 % of the kernel time of the timed evaluations, ahead of "
+                          "k_spread_z<1, false> (18.0 %), profiles/admp_12288_kernel_stats.md")
 
 
 def roofline(name, tm, D, prec, frames=1, prof=None):
@@ -605,6 +605,10 @@ def roofline(name, tm, D, prec, frames=1, prof=None):
       spread     N (3*8 + 4 w) + G w           positions, fractional charge+dipole, grid written once
       gather     G w + N 3*8 + N 3*8           grid, positions, field out
       real_matvec 2P (4 + 2 w) + N 3 (w + 8)   ELL index + two stored coefficients per ordered pair
+    Matrix-core path (no z launches of its own; at most the FP32 final pass has them):
+      spread     N (3*8 + 4 w) + 2 Gh w        half spectrum written once
+      gather     2 Gh w + N 3*8 + N 3*8        half spectrum, positions, field out
+      influence, plane_matvec as below
     FFT, fused plane path (two z launches per transform pair, one plane launch):
       fft        G w + 2 Gh w                  z R2C or C2R: real grid one way, half spectrum the other
       influence  4 Gh w + 8 Gh                 plane pass: half spectrum in and out, tabulated influence
@@ -613,7 +617,8 @@ def roofline(name, tm, D, prec, frames=1, prof=None):
       influence  4 Gh w + 8 Gh                 x pass: half spectrum in and out, tabulated influence
     plane_matvec (solver products with few frames: the plane pass and the real-space product in one launch)
                  4 Gh w + 8 Gh + 2P (4 + 2 w) + N 3 (w + 8)
-    The path is read off the launch counts: 2 or 4 fft launches per plane (influence or plane_matvec) launch.
+    The path is read off the launch counts: 2 or 4 fft launches per plane (influence or plane_matvec) launch, fewer
+    than one on the matrix-core path.
     """
     ms, n = tm
     t = ms / n / 1e3
@@ -625,18 +630,20 @@ def roofline(name, tm, D, prec, frames=1, prof=None):
     G = K[0] * K[1] * K[2]
     Gh = K[0] * K[1] * (K[2] // 2 + 1)
     P = D.get("n_pairs", 0)
-    plane = False
+    plane = mm = False
     n_plane = (prof.get("influence", (0, 0))[1] + prof.get("plane_matvec", (0, 0))[1]) if prof else 0
     if n_plane:
+        mm = prof.get("fft", (0, 0))[1] < n_plane
         plane = prof.get("fft", (0, 0))[1] < 3 * n_plane
+    grid = 2 * Gh * w if mm else G * w
     table = {
-        "spread": ("k_spread_cw", N * (3 * 8 + 4 * w) + G * w),
+        "spread": ("k_spread_z" if mm else "k_spread_cw", N * (3 * 8 + 4 * w) + grid),
         "fft": ("k_fz_r2c/k_fz_c2r", G * w + 2 * Gh * w) if plane else
                ("k_fz_r2c/k_fy/k_fz_c2r", (2 * G * w + 12 * Gh * w) / 4),
-        "influence": ("k_fxy_plane" if plane else "k_fx_infl", 4 * Gh * w + 8 * Gh),
-        "gather": ("k_gather_ml", G * w + N * 3 * 8 + N * 3 * 8),
+        "influence": ("k_plane_mm" if mm else "k_fxy_plane" if plane else "k_fx_infl", 4 * Gh * w + 8 * Gh),
+        "gather": ("k_gather_z" if mm else "k_gather_ml", grid + N * 3 * 8 + N * 3 * 8),
         "real_matvec": ("k_real_matvec", 2 * P * (4 + 2 * 8) + N * 3 * (8 + 8)),
-        "plane_matvec": ("k_plane_matvec", 4 * Gh * w + 8 * Gh + 2 * P * (4 + 2 * 8) + N * 3 * (8 + 8)),
+        "plane_matvec": ("k_plane_mm_matvec" if mm else "k_plane_matvec", 4 * Gh * w + 8 * Gh + 2 * P * (4 + 2 * 8) + N * 3 * (8 + 8)),
     }
     if name not in table or (name in ("real_matvec", "plane_matvec") and not P):
         return {"kernel": name, "bound": None, "achieved": None, "peak": None, "unit": None, "frac": None,
