@@ -442,6 +442,9 @@ if __name__ == "__main__":
     elif case == "polar_grid":
         from tests.systems import polar_grid
         out = {k: _lst(v) for k, v in polar_grid(tuple(int(k) for k in sys.argv[4].split(",")), "cpu").items()}
+    elif case == "jacobi_mixed":
+        from tests.systems import jacobi_mixed
+        out = {k: _lst(v) for k, v in jacobi_mixed("cpu").items()}
     elif case == "waters":
         out = waters(prec, int(sys.argv[4]))
     elif case == "frames" and len(sys.argv) > 4:

@@ -175,6 +175,13 @@ def test_matrix_core_grids_equal_radix_path(emu_lib, K):
         assert rel_rms(a[key], b[key]) < 1e-9, key
 
 
+def test_fp32_sweeps_keep_the_radix_right_hand_side(emu_lib):
+    """Jacobi sweeps with FP32 products follow the last bit of the right-hand side, so a mixed
+    context's FP64 passes stay on the radix path there: the same bits as when it is forced."""
+    a, b = (run(emu_lib, "jacobi_mixed", "mixed", extra_env=e) for e in (None, {"ADMP_SPREAD": "cw"}))
+    assert a == b
+
+
 def test_water_box_several_solver_blocks(emu_lib):
     """1,536 atoms: six solver blocks, the fused gather epilogue and a warm start."""
     r64 = run(emu_lib, "waters", "fp64", 512)
