@@ -134,7 +134,6 @@ struct admp_ctx {
     int* d_pcc = nullptr;       // the children, PC_MAXCH per site
     int pc_maxm = PC_MAXM;      // sites per preconditioner block (1: diagonal; admp_solver_opts.precond)
     CgCheck spread_chk{};       // convergence test of the next solver product (set by pcg_apply)
-    int* d_active = nullptr;
     int dots_blocks = 64;
     double* d_pparts = nullptr;               // CG partials (CgParts layout)
     int cg_nw = 0;                            // z.w slots per frame
@@ -786,7 +785,6 @@ extern "C" admp_status admp_ctx_create(const admp_config* cfg, admp_ctx** out) {
     ALLOC(ctx->d_eout, ctx->F);
     ALLOC(ctx->d_bout, (size_t)ctx->F * 9);
     ALLOC(ctx->d_coef, ctx->F * 4);
-    ALLOC(ctx->d_active, ctx->F);
     ALLOC(ctx->d_maxcnt, 1);
     ALLOC(ctx->d_geom, 1);
     ALLOC(ctx->d_cgflag, ctx->F);
@@ -1626,11 +1624,12 @@ static admp_status recip_run(admp_ctx* ctx, const Grid& g, int use_dA, const dou
     return ADMP_OK;
 }
 
-// A v for the induced-dipole system (everything but the right-hand side).
+// Parts of A v for the induced-dipole system but its diagonal: the real-space product into
+// ctx->d_t1 and the reciprocal one into *rec (null without PME).
 // RC: type of the stored pair coefficients; R: arithmetic of the real-space and
 // reciprocal products (the mixed solver's FP64 residual uses RC=float, R=double).
 template <class RC, class R>
-static admp_status matvec(admp_ctx* ctx, const double* v, double* out, const double* pol, double f1) {
+static admp_status products(admp_ctx* ctx, const double* v, const PcgState* skip, double** rec) {
     const int N = ctx->N, F = ctx->F;
     const size_t NF = (size_t)N * F;
     hipStream_t st = ctx->stream;
@@ -1645,14 +1644,26 @@ static admp_status matvec(admp_ctx* ctx, const double* v, double* out, const dou
     const int nbf = (int)nblk((size_t)N * TPA, PAIR_BLOCK);
     hipLaunchKernelGGL((k_real_matvec<RC, R, MatvecArrays<R>>), dim3(xcd_blocks(nbf * F)), dim3(PAIR_BLOCK), 0, st, N, nbf,
                        F, ctx->cap, ctx->d_box, ctx->d_nbr, ctx->d_ncnt, reinterpret_cast<const RC*>(ctx->d_pcoef),
-                       (MatvecArrays<R>{ctx->d_pos, vR}), ctx->d_t1, (const PcgState*)nullptr); }
-    double* rec = nullptr;
+                       (MatvecArrays<R>{ctx->d_pos, vR}), ctx->d_t1, skip); }
+    *rec = nullptr;
     if (ctx->cfg.lpme) {
         admp_status s = recip_run<R>(ctx, ctx->eg, 0, nullptr, v, 2, 1, 0, DIELECTRIC, ctx->cfg.kappa, 1, ctx->d_t2,
-                                     nullptr, nullptr, nullptr, false);
+                                     nullptr, nullptr, nullptr, false, nullptr, nullptr, skip);
         if (s != ADMP_OK) return s;
-        rec = ctx->d_t2;
+        *rec = ctx->d_t2;
     }
+    HIPCHK(hipGetLastError());
+    return ADMP_OK;
+}
+
+// A v for the induced-dipole system (everything but the right-hand side).
+template <class RC, class R>
+static admp_status matvec(admp_ctx* ctx, const double* v, double* out, const double* pol, double f1) {
+    const int N = ctx->N, F = ctx->F;
+    hipStream_t st = ctx->stream;
+    double* rec;
+    const admp_status s = products<RC, R>(ctx, v, nullptr, &rec);
+    if (s != ADMP_OK) return s;
     { ProfScope ps_(ctx, 11);
     hipLaunchKernelGGL(k_apply_diag, dim3(nblk(N, 256), F), dim3(256), 0, st, N, f1, pol, v, ctx->d_t1, rec, out); }
     HIPCHK(hipGetLastError());
@@ -2170,7 +2181,6 @@ static admp_status solve(admp_ctx* ctx, const double* pol, const double* thole, 
     info.n_iter.assign(F, 0);
     info.conv.assign(F, 0);
     info.res.assign(F, 0.0);
-    std::vector<int> act(F, 1);
     std::vector<double> h;
     // With FP64 products throughout, the CG's recursively updated residual (which
     // decides convergence) is what is reported: its drift from the true residual
@@ -2207,32 +2217,47 @@ static admp_status solve(admp_ctx* ctx, const double* pol, const double* thole, 
             return ADMP_OK;
         }
     } else {
-        // Jacobi sweeps (pme.py:380-422)
-        HIPCHK(hipMemcpyAsync(ctx->d_active, act.data(), F * sizeof(int), hipMemcpyHostToDevice, st));
-        int i = 0;
-        for (i = 0; i < maxiter; ++i) {
-            if ((s = matvec<double, R>(ctx, U, ctx->d_Ap, pol, f1)) != ADMP_OK) return s;
-            hipLaunchKernelGGL(k_sub, dim3(nblk(NF * 3, 256)), dim3(256), 0, st, NF * 3, ctx->d_b, ctx->d_Ap);
-            if (kind == ADMP_SOLVER_REFERENCE) {
-                if ((s = dots(ctx, ctx->d_Ap, nullptr, nullptr, pol, h)) != ADMP_OK) return s;
-                int nact = 0;
-                for (int f = 0; f < F; ++f) {
-                    if (act[f]) {
-                        info.res[f] = h[3 * f + 2];
-                        if (h[3 * f + 2] < tol) { act[f] = 0; info.conv[f] = 1; info.n_iter[f] = i; }
-                    }
-                    nact += act[f];
-                }
-                if (!nact) break;
-                HIPCHK(hipMemcpyAsync(ctx->d_active, act.data(), F * sizeof(int), hipMemcpyHostToDevice, st));
+        // Jacobi sweeps (pme.py:380-422).  The convergence test is on the device; the host
+        // reads the state of the sweep before while the next one runs, so that it stops
+        // launching one sweep late (whose kernels find their frames done).
+        const bool test = kind == ADMP_SOLVER_REFERENCE;
+        HIPCHK(hipMemsetAsync(ctx->d_pcg, 0, F * sizeof(PcgState), st));
+        std::vector<PcgState> hs(F);
+        memset(hs.data(), 0, F * sizeof(PcgState));
+        auto read = [&](int i) -> admp_status {
+            HIPCHK(hipEventSynchronize(ctx->ev_state[i & 1]));
+            std::copy(ctx->h_pcg + (size_t)(i & 1) * F, ctx->h_pcg + (size_t)(i & 1) * F + F, hs.begin());
+            return ADMP_OK;
+        };
+        bool all = false;
+        for (int i = 0; i < maxiter && !all; ++i) {
+            double* rec;
+            if ((s = products<double, R>(ctx, U, ctx->d_pcg, &rec)) != ADMP_OK) return s;
+            {
+                ProfScope ps_(ctx, 11);
+                const dim3 gr(nblk(N, 256), F);
+                hipLaunchKernelGGL(k_jacobi_grad, gr, dim3(256), 0, st, N, f1, pol, U, ctx->d_t1, rec, ctx->d_b, ctx->d_Ap,
+                                   ctx->d_pparts, ctx->d_pcg);
+                hipLaunchKernelGGL(k_jacobi, gr, dim3(256), 0, st, N, i, test ? tol : -1.0, pol, ctx->d_Ap, ctx->d_pparts, U,
+                                   ctx->d_pcg);
             }
-            hipLaunchKernelGGL(k_jacobi, dim3(nblk(N, 256), F), dim3(256), 0, st, N, ctx->d_active, pol, ctx->d_Ap, U);
+            if (!test) continue;
+            HIPCHK(hipMemcpyAsync(ctx->h_pcg + (size_t)(i & 1) * F, ctx->d_pcg, F * sizeof(PcgState),
+                                  hipMemcpyDeviceToHost, st));
+            HIPCHK(hipEventRecord(ctx->ev_state[i & 1], st));
+            if (i > 0) {
+                if ((s = read(i - 1)) != ADMP_OK) return s;
+                all = std::all_of(hs.begin(), hs.end(), [](const PcgState& p) { return p.done; });
+            }
         }
+        if (test && maxiter > 0 && !all && (s = read(maxiter - 1)) != ADMP_OK) return s;
         for (int f = 0; f < F; ++f) {
-            if (kind == ADMP_SOLVER_STEPS) { info.n_iter[f] = maxiter; info.conv[f] = 1; }
-            else if (act[f]) { info.n_iter[f] = maxiter - 1; info.conv[f] = 0; }
+            if (!test) { info.n_iter[f] = maxiter; info.conv[f] = 1; continue; }
+            info.res[f] = hs[f].res;
+            info.conv[f] = hs[f].done ? 1 : 0;
+            info.n_iter[f] = hs[f].done ? hs[f].iter : maxiter - 1;
         }
-        if (kind == ADMP_SOLVER_REFERENCE) {
+        if (test) {
             HIPCHK(hipGetLastError());
             return ADMP_OK;
         }

@@ -628,6 +628,37 @@ def test_pair_rows_in_any_order(n_pairs):
         assert all(np.array_equal(a, b) for a, b in zip(o, out[0]))
 
 
+@pytest.mark.parametrize("maxiter", [1, 2, 40])
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+def test_jacobi_frames_stop_alone(maxiter, prec):
+    """Jacobi sweeps of frames that converge after different numbers of sweeps, or not within
+    maxiter: sweep counts, flags, residuals and dipoles are those of each frame alone, bit by
+    bit (the same kernels on the same values)."""
+    from dmff_amd.admp.engine import Engine
+    s, pos, box = _small_waters()
+    rng = np.random.default_rng(23)
+    P = np.stack([pos + rng.normal(0, sg, pos.shape) for sg in (0.0, 0.02, 0.05)])
+    Q, pol, th = s.pme.Q_local[s.map_atomtype], s.pme.pol[s.map_poltype], s.pme.thole[s.map_poltype]
+
+    def run(Pf):
+        n = len(Pf)
+        eng = Engine(len(pos), 2, True, True, 0.4, (18, 19, 17), 6.0, n_frames=n, precision=prec, device=DEV)
+        eng.set_topology(s.axis_types, s.axis_idx, s.bonded)
+        eng.build_neighbors(Pf, np.stack([box] * n))
+        E, g, U, info = eng.compute(Pf, np.stack([box] * n), Q, pol, th, s.pme.mScales, s.pme.pScales, s.pme.dScales,
+                                    solver="reference", tol=0.5, maxiter=maxiter, want_grad=True)
+        return U.cpu().numpy(), info
+
+    U, info = run(P)
+    print(prec, maxiter, info["n_iter"], info["residual"], flush=True)
+    for k in range(3):
+        U1, i1 = run(P[k:k + 1])
+        assert info["n_iter"][k] == i1["n_iter"][0] and info["residual"][k] == i1["residual"][0]
+        assert np.array_equal(U[k], U1[0])
+        if maxiter < 3:
+            assert info["n_iter"][k] == maxiter - 1 and info["residual"][k] > 0.5
+
+
 def test_per_frame_pairs_survive_capacity_growth():
     """Pair lists set frame by frame, the second one longer (capacity grows):
     the first frame's list must survive the reallocation (dmff/utils.py:65-84
