@@ -129,9 +129,9 @@ struct PairParams {
 // gradients need stay; the gradients, which read the records again (from L2, and the own site's from LDS).
 // The virial differs from zero only for pairs across the boundary: its sums stay in LDS.
 // pair_step() ends a step for the compiler, which would otherwise load early and hold.
-// 225 registers' worth of values instead of 320, two wavefronts per SIMD, 753 FP64
-// instructions per pair instead of 906: 180 -> 155 us at 12,288 sites (90 neighbours each),
-// 10.4 -> 7.5 ms for 64 such frames.  Forcing three wavefronts spills 80 registers: 16 ms.
+// 212 registers instead of 320 (which is one wavefront per SIMD), 753 FP64 instructions per
+// pair instead of 906: 180 -> 145 us at 12,288 sites (215 neighbours each), 10.4 -> 7.2 ms
+// for 64 such frames.  Forcing three wavefronts spills 80 registers: 16 ms.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void pair_step(int& j) {
     __builtin_amdgcn_sched_barrier(0);

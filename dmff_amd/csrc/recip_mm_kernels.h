@@ -18,7 +18,7 @@
 // 1,536 sites on 25 x 25 x 25: 15.6 -> 9.4, 13.9 -> 10.4, 9.9 -> 7.7 us; 64 frames of 12,288
 // sites: level (1.85 ms).  On axes that are prime or hold a prime factor above 13 the radix
 // passes sum directly: for 2,970 sites r2c 74, plane 112 and c2r 70 us of each of eleven
-// sweeps, and the evaluation falls from 4.7 to 1.8 ms.
+// sweeps, and the evaluation falls from 4.7 to 1.8 ms (with the sweeps' test on the host).
 //
 // Fragments of v_mfma_f64_16x16x4 (lane l of the wavefront): A holds row l % 16,
 // column l / 16 of a 16 x 4 block, B row l / 16, column l % 16 of a 4 x 16 block, and
