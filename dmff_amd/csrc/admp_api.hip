@@ -99,6 +99,7 @@ struct admp_ctx {
     int *d_bcount = nullptr, *d_bstart = nullptr;  // per-brick candidate counts / offsets
     int2* d_blist = nullptr;                        // per-brick candidate lists
     double* d_infl = nullptr;                       // tabulated electrostatic influence function (eg)
+    double* d_dinfl = nullptr;                      // the dispersion kinds' and its derivative (dg), per pass
     int infl_pm = 0;                                // its layout: plane-major (1) or line-major (0)
     // a solve with FP32 products is running: its FP64 passes take the radix path (use_mm)
     bool radix64 = false;
@@ -420,8 +421,8 @@ static bool mm_kernels_ready() {
                            (const void*)k_gather_z<0>, (const void*)k_gather_z<1>, (const void*)k_gather_z<2>,
 #define ADMP_MM_NT(NTv)                                                                                               \
     (const void*)k_plane_mm<NTv, IN_TABLE>, (const void*)k_plane_mm<NTv, IN_TABLE_ACC>,                              \
-        (const void*)k_plane_mm<NTv, IN_ACC>, (const void*)k_plane_mm_matvec<NTv>, (const void*)k_y_mm<NTv>,          \
-        (const void*)k_x_mm<NTv, IN_TABLE>, (const void*)k_x_mm<NTv, IN_TABLE_ACC>, (const void*)k_x_mm<NTv, IN_ACC>
+        (const void*)k_plane_mm<NTv, IN_TABLE2_ACC>, (const void*)k_plane_mm_matvec<NTv>, (const void*)k_y_mm<NTv>,          \
+        (const void*)k_x_mm<NTv, IN_TABLE>, (const void*)k_x_mm<NTv, IN_TABLE_ACC>, (const void*)k_x_mm<NTv, IN_TABLE2_ACC>
                            ADMP_MM_NT(1), ADMP_MM_NT(2), ADMP_MM_NT(3), ADMP_MM_NT(4), ADMP_MM_NT(5)};
 #undef ADMP_MM_NT
         static_assert(MM_NT == 5, "one instance per number of row tiles");
@@ -754,6 +755,8 @@ extern "C" admp_status admp_ctx_create(const admp_config* cfg, admp_ctx** out) {
         }
         if (ctx->eg.G)
             ALLOC(ctx->d_infl, (size_t)ctx->eg.K[0] * ctx->eg.K[1] * (ctx->eg.K[2] / 2 + 1) * ctx->F);
+        if (ctx->dg.mm)
+            ALLOC(ctx->d_dinfl, 2 * (size_t)ctx->dg.K[0] * ctx->dg.K[1] * (ctx->dg.K[2] / 2 + 1) * ctx->F);
     }
     ALLOC(ctx->d_wd, NF * 3);
     ALLOC(ctx->d_gcell, NF);
@@ -1334,9 +1337,18 @@ static admp_status recip_run_mm(admp_ctx* ctx, const Grid& g, int use_dA, const 
     if ((s = run_after_spread(ctx)) != ADMP_OK) return s;
     const bool use_tab = &g == &ctx->eg && kind == 0 && !use_dA && pref == DIELECTRIC && kappa == ctx->cfg.kappa &&
                          ctx->d_infl && ctx->infl_pm;
-    const InflArgs q{ctx->d_box, g.bmod[0], g.bmod[1], g.bmod[2], kappa, kind, pref, ctx->d_infl, ctx->d_part};
-    // without the table (another grid or kind than the solver's) the function is computed
-    const int in = !use_tab ? IN_ACC : want_energy ? IN_TABLE_ACC : IN_TABLE;
+    // the electrostatic function is tabulated once per evaluation, a dispersion kind's for its pass
+    const int in = !use_tab ? IN_TABLE2_ACC : want_energy ? IN_TABLE_ACC : IN_TABLE;
+    double* tabd = nullptr;
+    if (!use_tab) {
+        if (!ctx->d_dinfl || &g != &ctx->dg) { ctx->err = "no influence table for this grid"; return ADMP_ERR_STATE; }
+        ProfScope ps_(ctx, 6);
+        tabd = ctx->d_dinfl + (size_t)K0 * K1 * H * F;
+        hipLaunchKernelGGL(k_infl_table2, dim3(nblk((size_t)K0 * K1 * H, 256), F), dim3(256), 0, st, K0, K1, K2, ctx->d_box,
+                           g.bmod[0], g.bmod[1], g.bmod[2], kappa, kind, pref, ctx->d_dinfl, tabd);
+    }
+    const InflArgs q{ctx->d_box, g.bmod[0], g.bmod[1], g.bmod[2], kappa, kind, pref, use_tab ? ctx->d_infl : ctx->d_dinfl,
+                     tabd, ctx->d_part};
     const int ntx = mm_tiles(K0), nty = mm_tiles(K1);
     int npart = H;
     // f(row tiles) with the row tiles as a constant
@@ -1367,7 +1379,7 @@ static admp_status recip_run_mm(admp_ctx* ctx, const Grid& g, int use_dA, const 
                 hipLaunchKernelGGL((k_plane_mm<NT, IN_TABLE_ACC>), dim3(H, F), dim3(th), sm, st, K0, K1, K2, tx, ty, hg, q,
                                    skip);
             } else {
-                hipLaunchKernelGGL((k_plane_mm<NT, IN_ACC>), dim3(H, F), dim3(th), sm, st, K0, K1, K2, tx, ty, hg, q, skip);
+                hipLaunchKernelGGL((k_plane_mm<NT, IN_TABLE2_ACC>), dim3(H, F), dim3(th), sm, st, K0, K1, K2, tx, ty, hg, q, skip);
             }
         });
     } else {
@@ -1395,7 +1407,7 @@ static admp_status recip_run_mm(admp_ctx* ctx, const Grid& g, int use_dA, const 
                 else if (in == IN_TABLE_ACC)
                     hipLaunchKernelGGL((k_x_mm<NT, IN_TABLE_ACC>), gr, bl, sm, st, K0, K1, K2, tx, hg, q, skip);
                 else
-                    hipLaunchKernelGGL((k_x_mm<NT, IN_ACC>), gr, bl, sm, st, K0, K1, K2, tx, hg, q, skip);
+                    hipLaunchKernelGGL((k_x_mm<NT, IN_TABLE2_ACC>), gr, bl, sm, st, K0, K1, K2, tx, hg, q, skip);
             });
         }
         ylines(1);

@@ -387,7 +387,7 @@ k_spread_z(int N, int K0, int K1, int K2, int wpt, const Cplx<double>* __restric
 // written.
 // ---------------------------------------------------------------------------
 struct NoHook {
-    static constexpr bool ROLL = false, PRE = false;
+    static constexpr bool PRE = false;
     __device__ double pre(int, int) const { return 0.0; }
     __device__ double out(double v, double, int, int) { return v; }
 };
@@ -456,31 +456,17 @@ __device__ __forceinline__ void mm_lines(Cplx<double>* P, int K, int nl, int ls,
         const bool live = line < nl;
 #pragma unroll
         for (int m = 0; m < NT; ++m) {
-            if constexpr (Hook::ROLL) {
-                // a long out(): one copy of it per row tile, eight values in turn
-#pragma unroll 1
-                for (int v = 0; v < 8; ++v) {
-                    const int r = v >> 1;
-                    const double sr = r == 0 ? S[m][0] : r == 1 ? S[m][1] : r == 2 ? S[m][2] : S[m][3];
-                    const double c = r == 0 ? C[m][0] : r == 1 ? C[m][1] : r == 2 ? C[m][2] : C[m][3];
-                    const double s = sg * swap_pair(sr);
-                    const int k = m * 16 + 4 * r + k4, ko = v & 1 ? K - k : k;
-                    if (live && k < H && (!(v & 1) || (k > 0 && 2 * k < K)))
-                        d[2 * ko * es] = hook.out(v & 1 ? c - s : c + s, 0.0, line, ko);
-                }
-            } else {
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const double s = sg * swap_pair(S[m][r]), c = C[m][r];
-                    const int k = m * 16 + 4 * r + k4;
-                    if (live && k < H) {
-                        if (Hook::PRE && NT > 3) {
-                            pk[m][r] = hook.pre(line, k);
-                            pm[m][r] = hook.pre(line, k > 0 ? K - k : 0);
-                        }
-                        d[2 * k * es] = hook.out(c + s, pk[m][r], line, k);
-                        if (k > 0 && 2 * k < K) d[2 * (K - k) * es] = hook.out(c - s, pm[m][r], line, K - k);
+            for (int r = 0; r < 4; ++r) {
+                const double s = sg * swap_pair(S[m][r]), c = C[m][r];
+                const int k = m * 16 + 4 * r + k4;
+                if (live && k < H) {
+                    if (Hook::PRE && NT > 3) {
+                        pk[m][r] = hook.pre(line, k);
+                        pm[m][r] = hook.pre(line, k > 0 ? K - k : 0);
                     }
+                    d[2 * k * es] = hook.out(c + s, pk[m][r], line, k);
+                    if (k > 0 && 2 * k < K) d[2 * (K - k) * es] = hook.out(c - s, pm[m][r], line, K - k);
                 }
             }
         }
@@ -503,57 +489,65 @@ struct InflArgs {
     int kind;
     double pref;
     const double* tab;    // tabulated 2 pref C_k / theta_k^2, plane-major
-    double* part;         // energy and box partials, 7 per block (IN_ACC, IN_TABLE_ACC)
+    const double* tabd;   // pref (dC / d(k^2)) / theta_k^2 (IN_TABLE2_ACC)
+    double* part;         // energy and box partials, 7 per block (IN_TABLE_ACC, IN_TABLE2_ACC)
 };
 // influence function applied to one component of a spectrum.  IN_TABLE: the tabulated
 // electrostatic function (solver products).  IN_TABLE_ACC: the same with the energy
 // and box-derivative sums, which follow from the table: C = tab theta^2 / (2 pref) and
-// dC / d(k^2) = -C (1 / k^2 + 1 / (4 kappa^2)).  IN_ACC: computed, with the sums (the
-// dispersion kinds).
-enum { IN_TABLE = 0, IN_ACC = 1, IN_TABLE_ACC = 2 };
+// dC / d(k^2) = -C (1 / k^2 + 1 / (4 kappa^2)).  IN_TABLE2_ACC: the sums with the derivative
+// from a table of its own (the dispersion kinds; k_infl_table2).
+enum { IN_TABLE = 0, IN_TABLE2_ACC = 1, IN_TABLE_ACC = 2 };
+
+// Both tables of a dispersion kind.  Their exp and erfc are formed here by every CU at once:
+// in the plane pass, on the one CU a plane has, they took 21 of its 49 us (8,580 sites); the
+// table takes 3.4 us and the pass 28.
+__global__ void __launch_bounds__(256)
+k_infl_table2(int K0, int K1, int K2, const BoxInfo* __restrict__ boxes, const double* __restrict__ bmod0,
+              const double* __restrict__ bmod1, const double* __restrict__ bmod2, double kappa, int kind, double pref,
+              double* __restrict__ tab, double* __restrict__ tabd) {
+    const int f = blockIdx.y, H = K2 / 2 + 1, P = K0 * K1;
+    const int idx = blockIdx.x * 256 + threadIdx.x;
+    if (idx >= P * H) return;
+    const int i2 = idx / P, r = idx - i2 * P, i0 = r / K1, i1 = r - i0 * K1;
+    const InflPt q = infl_point(boxes[f], K0, K1, K2, i0, i1, i2, kappa, kind);
+    const double th = bmod0[i0] * bmod1[i1] * bmod2[i2];
+    const double ith2 = 1.0 / (th * th);
+    tab[(size_t)f * P * H + idx] = 2.0 * pref * q.C * ith2;
+    tabd[(size_t)f * P * H + idx] = pref * q.dC * ith2;
+}
+
 template <int KIND> struct InflHook {
-    static constexpr bool ROLL = KIND == IN_ACC, PRE = KIND != IN_ACC;
     const InflArgs& q;
     const BoxInfo& b;
     const double* tp;     // the plane of the table
+    const double* td;     // and of its derivative's
     int K0, K1, K2, y0, i2;
     bool on;              // off: values pass unchanged
     double sum[KIND == IN_TABLE ? 1 : 7];
-    __device__ __forceinline__ double pre(int line, int i0) const {
-        return KIND != IN_ACC && on ? tp[i0 * K1 + y0 + line] : 1.0;
-    }
+    static constexpr bool PRE = true;
+    __device__ __forceinline__ double pre(int line, int i0) const { return on ? tp[i0 * K1 + y0 + line] : 1.0; }
     __device__ __forceinline__ double out(double v, double t, int line, int i0) {
-        if constexpr (KIND == IN_TABLE) {
-            return v * t;
-        } else if constexpr (KIND == IN_TABLE_ACC) {
-            if (on) {
-                const int i1 = y0 + line;
-                const int m0 = i0 < (K0 + 1) / 2 ? i0 : i0 - K0, m1 = i1 < (K1 + 1) / 2 ? i1 : i1 - K1;
-                const int m2 = i2 < (K2 + 1) / 2 ? i2 : i2 - K2;
-                const double kx = b.kb[0] * m0 + b.kb[1] * m1 + b.kb[2] * m2;
-                const double ky = b.kb[3] * m0 + b.kb[4] * m1 + b.kb[5] * m2;
-                const double kz = b.kb[6] * m0 + b.kb[7] * m1 + b.kb[8] * m2;
-                const double ksq = kx * kx + ky * ky + kz * kz;
-                const double e = 0.5 * t * v * v * ((i2 == 0 || 2 * i2 == K2) ? 1.0 : 2.0);
-                const double wd = ksq > 0.0 ? e * (1.0 / ksq + 1.0 / (4.0 * q.kappa * q.kappa)) : 0.0;
-                sum[0] += e;
-                sum[1] += wd * kx * kx; sum[2] += wd * ky * ky; sum[3] += wd * kz * kz;
-                sum[4] += wd * kx * ky; sum[5] += wd * kx * kz; sum[6] += wd * ky * kz;
-            }
-            return v * t;
-        } else {
-            if (!on) return v;
+        if (KIND != IN_TABLE && on) {
             const int i1 = y0 + line;
-            const InflPt p = infl_point(b, K0, K1, K2, i0, i1, i2, q.kappa, q.kind);
-            const double th = q.bmod0[i0] * q.bmod1[i1] * q.bmod2[i2];
-            const double ith2 = 1.0 / (th * th);
-            const double w = q.pref * v * v * ith2 * ((i2 == 0 || 2 * i2 == K2) ? 1.0 : 2.0);
-            sum[0] += w * p.C;
-            const double wd = -w * p.dC;
-            sum[1] += wd * p.kx * p.kx; sum[2] += wd * p.ky * p.ky; sum[3] += wd * p.kz * p.kz;
-            sum[4] += wd * p.kx * p.ky; sum[5] += wd * p.kx * p.kz; sum[6] += wd * p.ky * p.kz;
-            return v * (2.0 * q.pref * p.C * ith2);
+            const int m0 = i0 < (K0 + 1) / 2 ? i0 : i0 - K0, m1 = i1 < (K1 + 1) / 2 ? i1 : i1 - K1;
+            const int m2 = i2 < (K2 + 1) / 2 ? i2 : i2 - K2;
+            const double kx = b.kb[0] * m0 + b.kb[1] * m1 + b.kb[2] * m2;
+            const double ky = b.kb[3] * m0 + b.kb[4] * m1 + b.kb[5] * m2;
+            const double kz = b.kb[6] * m0 + b.kb[7] * m1 + b.kb[8] * m2;
+            const double v2 = v * v * ((i2 == 0 || 2 * i2 == K2) ? 1.0 : 2.0), e = 0.5 * t * v2;
+            double wd;
+            if constexpr (KIND == IN_TABLE2_ACC) {
+                wd = -td[i0 * K1 + i1] * v2;
+            } else {
+                const double ksq = kx * kx + ky * ky + kz * kz;
+                wd = ksq > 0.0 ? e * (1.0 / ksq + 1.0 / (4.0 * q.kappa * q.kappa)) : 0.0;
+            }
+            sum[0] += e;
+            sum[1] += wd * kx * kx; sum[2] += wd * ky * ky; sum[3] += wd * kz * kz;
+            sum[4] += wd * kx * ky; sum[5] += wd * kx * kz; sum[6] += wd * ky * kz;
         }
+        return v * t;
     }
 };
 
@@ -600,8 +594,8 @@ __device__ __forceinline__ void plane_mm_body(int f, int i2, int nplane, int K0,
     __syncthreads();
     // forward y, forward x with the influence function, inverse x, inverse y: one copy
     // of the code
-    InflHook<KIND> infl{q, q.boxes[f], KIND == IN_ACC ? nullptr : q.tab + ((size_t)f * H + i2) * P,
-                        K0, K1, K2, 0, i2, false, {}};
+    const size_t to = ((size_t)f * H + i2) * P;
+    InflHook<KIND> infl{q, q.boxes[f], q.tab + to, KIND == IN_TABLE2_ACC ? q.tabd + to : nullptr, K0, K1, K2, 0, i2, false, {}};
 #pragma unroll 1
     for (int t = 0; t < 4; ++t) {
         const bool x = t == 1 || t == 2;
@@ -698,8 +692,8 @@ k_x_mm(int K0, int K1, int K2, const Cplx<double>* __restrict__ twx, Cplx<double
         if (y < nl) b0[x * es + y] = hg[(size_t)x * K1 + y];
     }
     __syncthreads();
-    InflHook<KIND> infl{q, q.boxes[f], KIND == IN_ACC ? nullptr : q.tab + ((size_t)f * H + i2) * K0 * K1,
-                        K0, K1, K2, y0, i2, false, {}};
+    const size_t to = ((size_t)f * H + i2) * K0 * K1;
+    InflHook<KIND> infl{q, q.boxes[f], q.tab + to, KIND == IN_TABLE2_ACC ? q.tabd + to : nullptr, K0, K1, K2, y0, i2, false, {}};
 #pragma unroll 1
     for (int t = 0; t < 2; ++t) {
         infl.on = t == 0;
