@@ -161,7 +161,9 @@ struct admp_ctx {
         hipGraphExec_t exec = nullptr;
         std::string key, seen;
     };
-    PhaseGraph g_setup, g_final;
+    // the final pass of a mixed context holds the build of its brick lists (g_final[0]) unless
+    // the solve has built them ([1]: FP32 products)
+    PhaseGraph g_setup, g_final[2];
     bool use_graphs = true;   // ADMP_NO_GRAPH=1 runs the chunk and phase launches eagerly
     double* d_pol = nullptr;  // context-owned copies of the caller's inputs (stable graph arguments):
     double* d_thole = nullptr;  // polarisabilities, Thole widths, local multipoles
@@ -190,7 +192,7 @@ static void clear_chunk_graphs(admp_ctx* ctx) {
 
 static void clear_graphs(admp_ctx* ctx) {
     clear_chunk_graphs(ctx);
-    for (admp_ctx::PhaseGraph* g : {&ctx->g_setup, &ctx->g_final}) {
+    for (admp_ctx::PhaseGraph* g : {&ctx->g_setup, &ctx->g_final[0], &ctx->g_final[1]}) {
         if (g->exec) (void)hipGraphExecDestroy(g->exec);
         *g = admp_ctx::PhaseGraph();
     }
@@ -2392,11 +2394,15 @@ static admp_status compute_impl(admp_ctx* ctx, const double* Q_local, const doub
     return ADMP_OK;
     };
     if (lpol && lpme) {
-        // graph key: every value the captured launches take by value
+        // graph key: every value the captured launches take by value, and the host state
+        // that decides which launches there are (the sort and the lists that the solve left)
         std::string key;
         key_add(key, want_grad);
         key_add(key, pp);
-        if ((s = run_phase(ctx, ctx->g_final, key, final_body)) != ADMP_OK) return s;
+        key_add(key, ctx->prepped == &ctx->eg);
+        key_add(key, ctx->tiles_ok);
+        key_add(key, ctx->bricks_ok);
+        if ((s = run_phase(ctx, ctx->g_final[ctx->bricks_ok], key, final_body)) != ADMP_OK) return s;
     } else if ((s = final_body()) != ADMP_OK) {
         return s;
     }

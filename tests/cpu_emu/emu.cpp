@@ -249,16 +249,28 @@ void run_block(void (*entry)(void*), void* arg, unsigned bx, unsigned by, unsign
 }  // namespace emu
 
 // ------------------------------------------------------------------ runtime
+// Operations run at once, in the order of the calls, whatever their stream; between the
+// begin and the end of a capture they are recorded instead (arguments by value) and run
+// at every launch of the graph.
+struct emu_graph { std::vector<std::function<void()>> ops; };
+struct emu_graph_exec { emu_graph g; };
+static emu_graph* g_capture = nullptr;
+namespace emu {
+void submit(std::function<void()> op) {
+    if (g_capture) g_capture->ops.push_back(std::move(op));
+    else op();
+}
+}  // namespace emu
 struct emu_stream { int x; };
 struct emu_event { int x; };
 hipError_t hipMallocAsync(void** p, size_t bytes, hipStream_t) { *p = emu::galloc(bytes); return *p ? hipSuccess : 2; }
 hipError_t hipMalloc(void** p, size_t bytes) { return hipMallocAsync(p, bytes, nullptr); }
 hipError_t hipFreeAsync(void* p, hipStream_t) { emu::gfree(p); return hipSuccess; }
 hipError_t hipFree(void* p) { emu::gfree(p); return hipSuccess; }
-hipError_t hipMemsetAsync(void* p, int v, size_t n, hipStream_t) { memset(p, v, n); return hipSuccess; }
-hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) { memmove(d, s, n); return hipSuccess; }
+hipError_t hipMemsetAsync(void* p, int v, size_t n, hipStream_t) { emu::submit([=] { memset(p, v, n); }); return hipSuccess; }
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) { emu::submit([=] { memmove(d, s, n); }); return hipSuccess; }
 hipError_t hipMemcpy2DAsync(void* d, size_t dp, const void* s, size_t sp, size_t w, size_t h, hipMemcpyKind, hipStream_t) {
-    for (size_t r = 0; r < h; ++r) memmove((char*)d + r * dp, (const char*)s + r * sp, w);
+    emu::submit([=] { for (size_t r = 0; r < h; ++r) memmove((char*)d + r * dp, (const char*)s + r * sp, w); });
     return hipSuccess;
 }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
@@ -279,9 +291,20 @@ const char* hipGetErrorString(hipError_t) { return "emu error"; }
 hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
 hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { *v = 163840; return hipSuccess; }
 hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { return hipSuccess; }
-hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipErrorNotSupported; }
-hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t* g) { *g = nullptr; return hipErrorNotSupported; }
-hipError_t hipGraphInstantiate(hipGraphExec_t*, hipGraph_t, void*, void*, size_t) { return hipErrorNotSupported; }
-hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipErrorNotSupported; }
-hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
-hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) {
+    if (g_capture) return hipErrorInvalidValue;
+    g_capture = new emu_graph();
+    return hipSuccess;
+}
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t* g) {
+    *g = g_capture;
+    g_capture = nullptr;
+    return *g ? hipSuccess : hipErrorInvalidValue;
+}
+hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t g, void*, void*, size_t) { *e = new emu_graph_exec{*g}; return hipSuccess; }
+hipError_t hipGraphLaunch(hipGraphExec_t e, hipStream_t) {
+    for (auto& op : e->g.ops) op();
+    return hipSuccess;
+}
+hipError_t hipGraphDestroy(hipGraph_t g) { delete g; return hipSuccess; }
+hipError_t hipGraphExecDestroy(hipGraphExec_t e) { delete e; return hipSuccess; }

@@ -9,6 +9,8 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
+#include <memory>
 #include <unistd.h>
 #include <tuple>
 #include <type_traits>
@@ -52,6 +54,7 @@ void* dyn_smem();
 void begin_kernel(const char* name, dim3 g, dim3 b, size_t smem);
 void run_block(void (*entry)(void*), void* arg, unsigned bx, unsigned by, unsigned bz);
 void end_kernel();
+void submit(std::function<void()> op);   // runs it, or records it into the graph being captured
 template <class T> long long to_bits(T v) { long long r = 0; std::memcpy(&r, &v, sizeof(T)); return r; }
 template <class T> T from_bits(long long b) { T r; std::memcpy(&r, &b, sizeof(T)); return r; }
 }  // namespace emu
@@ -161,16 +164,18 @@ template <class... KA, class... A>
 void launch(const char* name, void (*k)(KA...), dim3 g, dim3 b, size_t smem, A&&... a) {
     using Tup = std::tuple<typename std::decay<KA>::type...>;
     struct Pack { void (*k)(KA...); Tup args; };
-    Pack pk{k, Tup(std::forward<A>(a)...)};
+    auto pk = std::make_shared<Pack>(Pack{k, Tup(std::forward<A>(a)...)});
     auto entry = [](void* p) {
         Pack* q = static_cast<Pack*>(p);
         std::apply(q->k, q->args);
     };
-    begin_kernel(name, g, b, smem);
-    for (unsigned z = 0; z < g.z; ++z)
-        for (unsigned y = 0; y < g.y; ++y)
-            for (unsigned x = 0; x < g.x; ++x) run_block(entry, &pk, x, y, z);
-    end_kernel();
+    submit([=] {
+        begin_kernel(name, g, b, smem);
+        for (unsigned z = 0; z < g.z; ++z)
+            for (unsigned y = 0; y < g.y; ++y)
+                for (unsigned x = 0; x < g.x; ++x) run_block(entry, pk.get(), x, y, z);
+        end_kernel();
+    });
 }
 }  // namespace emu
 #define hipLaunchKernelGGL(F, G, B, S, ST, ...) emu::launch(#F, F, dim3(G), dim3(B), (size_t)(S), ##__VA_ARGS__)

@@ -445,6 +445,10 @@ if __name__ == "__main__":
     elif case == "jacobi_mixed":
         from tests.systems import jacobi_mixed
         out = {k: _lst(v) for k, v in jacobi_mixed("cpu").items()}
+    elif case == "solver_sequence":
+        from tests.systems import SOLVER_SEQUENCES, solver_sequence
+        out = [[_lst(x) for x in call]
+               for call in solver_sequence(*SOLVER_SEQUENCES[int(sys.argv[4])], "cpu", prec == "fresh")]
     elif case == "waters":
         out = waters(prec, int(sys.argv[4]))
     elif case == "frames" and len(sys.argv) > 4:

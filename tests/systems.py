@@ -336,6 +336,35 @@ def jacobi_mixed(device):
     return {"E": E.cpu().numpy(), "U": U.cpu().numpy(), "pos": g["pos"].cpu().numpy()}
 
 
+# solver kinds of the calls on one mixed context
+SOLVER_SEQUENCES = [((18, 19, 17), "reference reference pcg pcg"), ((18, 19, 17), "pcg steps pcg steps"),
+                    ((18, 19, 17), "pcg fp32 pcg warm fp32")]
+
+
+def solver_sequence(K, sequence, device, fresh):
+    """The calls of a sequence, each on other positions and one tighter in tolerance (so that
+    new lengths of solver chunks come up), by one mixed context or by a new one each: energy,
+    force and dipoles of every call."""
+    from dmff_amd.admp.engine import Engine
+    s, pos, box = small_water_box()
+    rng = np.random.default_rng(29)
+    out, eng = [], None
+    for n, kind in enumerate(sequence.split()):
+        if fresh or eng is None:
+            eng = Engine(len(pos), 2, True, True, 0.4, K, 6.0, precision="mixed", device=device)
+            eng.set_topology(s.axis_types, s.axis_idx, s.bonded)
+        p = pos + 0.7 * n + rng.normal(0, 0.03, pos.shape)
+        eng.build_neighbors(p, box)
+        solver = kind if kind in ("reference", "steps") else "pcg"
+        U0 = np.zeros((1, len(pos), 3)) if kind == "warm" else None
+        E, g, U, info = eng.compute(p, box, s.pme.Q_local[s.map_atomtype], s.pme.pol[s.map_poltype],
+                                    s.pme.thole[s.map_poltype], s.pme.mScales, s.pme.pScales, s.pme.dScales, U_init=U0,
+                                    solver=solver, tol=0.5 if kind == "reference" else 1e-4, maxiter=50, steps=3,
+                                    fp32_products=kind == "fp32", want_grad=True)
+        out.append([x.detach().cpu().numpy().ravel() for x in (E, g["pos"], g["box"], U)])
+    return out
+
+
 def polar_grid_oracle(K):
     """Frame 0 of polar_grid by the oracle."""
     import torch

@@ -22,7 +22,7 @@ import pytest
 import torch
 
 from oracle import admp_oracle as O
-from tests.systems import MATRIX_GRIDS, reference_pairs, small_water_box
+from tests.systems import MATRIX_GRIDS, SOLVER_SEQUENCES, reference_pairs, small_water_box
 from tests.test_gpu_parity import compare, oracle_eval, rel_rms
 
 REPO = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -180,6 +180,16 @@ def test_fp32_sweeps_keep_the_radix_right_hand_side(emu_lib):
     context's FP64 passes stay on the radix path there: the same bits as when it is forced."""
     a, b = (run(emu_lib, "jacobi_mixed", "mixed", extra_env=e) for e in (None, {"ADMP_SPREAD": "cw"}))
     assert a == b
+
+
+@pytest.mark.parametrize("case", range(len(SOLVER_SEQUENCES)))
+def test_solver_kinds_in_turn_on_one_context(emu_lib, case):
+    """Calls with different solvers on one mixed context, whose phases are captured and replayed:
+    each equals, bit by bit, the same call on a new context, which runs everything eagerly (the
+    same kernels on the same values)."""
+    a, b = (run(emu_lib, "solver_sequence", how, case) for how in ("one", "fresh"))
+    for n, (x, y) in enumerate(zip(a, b)):
+        assert x == y, (SOLVER_SEQUENCES[case], n)
 
 
 def test_water_box_several_solver_blocks(emu_lib):

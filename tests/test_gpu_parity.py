@@ -12,7 +12,8 @@ import pytest
 import torch
 
 from oracle import admp_oracle as O
-from tests.systems import MATRIX_GRIDS, load_system, polar_grid, polar_grid_oracle, reference_pairs, small_water_box as _small_waters
+from tests.systems import (MATRIX_GRIDS, SOLVER_SEQUENCES, load_system, polar_grid, polar_grid_oracle, reference_pairs,
+                           small_water_box as _small_waters, solver_sequence)
 
 pytestmark = pytest.mark.gpu
 F64 = torch.float64
@@ -602,6 +603,16 @@ def test_matrix_core_grids(K):
     errs = {k: rel_rms(a[k][0], o[k]) for k in o}
     print(f"K={K}: {errs}", flush=True)
     assert errs.pop("E") < 1e-9 and max(errs.values()) < 1e-7
+
+
+@pytest.mark.parametrize("case", range(len(SOLVER_SEQUENCES)))
+def test_solver_kinds_in_turn_on_one_context(case):
+    """Calls with different solvers on one mixed context, whose phases are captured and replayed:
+    each equals, bit by bit, the same call on a new context, which runs everything eagerly."""
+    K, sequence = SOLVER_SEQUENCES[case]
+    a, b = (solver_sequence(K, sequence, DEV, fresh) for fresh in (False, True))
+    for n, (x, y) in enumerate(zip(a, b)):
+        assert all(np.array_equal(u, v) for u, v in zip(x, y)), (K, sequence, n)
 
 
 @pytest.mark.parametrize("n_pairs", [1, 63, 64, 65, 257, None])
