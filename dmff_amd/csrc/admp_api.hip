@@ -1224,6 +1224,10 @@ static admp_status admp_get_pairs_impl(admp_ctx* ctx, int32_t frame, int32_t* ou
 // axis has at least brick + 5 points; smaller grids take the scatter path.
 static bool small_grid(const Grid& g) { return g.K[0] < BRX + 5 || g.K[1] < BRY + 5 || g.K[2] < BRZ + 5; }
 
+// layout of the electrostatic influence table: that of the FP64 solver products' passes
+// (plane-major: 1), which differ between solves of a mixed context (use_mm)
+static int infl_layout(const admp_ctx* ctx) { return use_mm(ctx, ctx->eg) || ctx->eg.plane[1] ? 1 : 0; }
+
 static admp_status recip_positions(admp_ctx* ctx, const Grid& g, int use_dA) {
     const int N = ctx->N, F = ctx->F;
     hipStream_t st = ctx->stream;
@@ -1245,8 +1249,7 @@ static admp_status recip_positions(admp_ctx* ctx, const Grid& g, int use_dA) {
                            ctx->d_gcatoms);
         if (&g == &ctx->eg && ctx->d_infl && !use_dA) {
             const size_t nt = (size_t)g.K[0] * g.K[1] * (g.K[2] / 2 + 1);
-            // laid out for the FP64 solver products' FFT path
-            ctx->infl_pm = use_mm(ctx, g) || g.plane[1] ? 1 : 0;
+            ctx->infl_pm = infl_layout(ctx);
             hipLaunchKernelGGL(k_infl_table, dim3(nblk(nt, 256), F), dim3(256), 0, st, g.K[0], g.K[1], g.K[2],
                                ctx->d_box, g.bmod[0], g.bmod[1], g.bmod[2], ctx->cfg.kappa, DIELECTRIC, ctx->infl_pm,
                                ctx->d_infl);
@@ -2182,10 +2185,12 @@ static admp_status solve(admp_ctx* ctx, const double* pol, const double* thole, 
             return pcg_restart<double>(ctx, ctx->d_b, U, pol, f1, tol, 1, true, true, U);
         });
         if (s != ADMP_OK) return s;
-        // a replayed set-up graph sorted the sites for the spread as well (the host
-        // state its capture left): later launches and captures must not sort again
+        // a replayed set-up graph sorted the sites for the spread as well and laid out the
+        // influence table (the host state its capture left): later launches and captures
+        // must not sort again, and read the table as it is now
         if (c.lpme) {
             ctx->prepped = &ctx->eg;
+            ctx->infl_pm = infl_layout(ctx);
             (use_mm(ctx, ctx->eg) ? ctx->tiles_ok : ctx->bricks_ok) = true;
         }
     } else {

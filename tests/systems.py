@@ -336,9 +336,11 @@ def jacobi_mixed(device):
     return {"E": E.cpu().numpy(), "U": U.cpu().numpy(), "pos": g["pos"].cpu().numpy()}
 
 
-# solver kinds of the calls on one mixed context
+# solver kinds of the calls on one mixed context, on a grid whose FP64 plane fits the radix
+# plane pass and on one past it, where the influence table has either layout by turns
 SOLVER_SEQUENCES = [((18, 19, 17), "reference reference pcg pcg"), ((18, 19, 17), "pcg steps pcg steps"),
-                    ((18, 19, 17), "pcg fp32 pcg warm fp32")]
+                    ((18, 19, 17), "pcg fp32 pcg warm fp32"), ((64, 64, 9), "pcg pcg steps pcg"),
+                    ((64, 64, 9), "steps pcg pcg fp32 pcg")]
 
 
 def solver_sequence(K, sequence, device, fresh):
