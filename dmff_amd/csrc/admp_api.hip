@@ -274,6 +274,10 @@ static admp_status run_phase(admp_ctx* ctx, admp_ctx::PhaseGraph& pg, const std:
         (void)hipGraphExecDestroy(pg.exec);
         pg.exec = nullptr;
     }
+    // host state that the body's launches change, should the capture come to nothing
+    const Grid* prepped = ctx->prepped;
+    const bool bricks_ok = ctx->bricks_ok, tiles_ok = ctx->tiles_ok;
+    const int infl_pm = ctx->infl_pm;
     hipGraph_t graph = nullptr;
     if (hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal) != hipSuccess) {
         (void)hipGetLastError();
@@ -288,6 +292,10 @@ static admp_status run_phase(admp_ctx* ctx, admp_ctx::PhaseGraph& pg, const std:
     if (ie != hipSuccess) {
         // nothing of the capture ran: report the body's error, or run it eagerly
         (void)hipGetLastError();
+        ctx->prepped = prepped;
+        ctx->bricks_ok = bricks_ok;
+        ctx->tiles_ok = tiles_ok;
+        ctx->infl_pm = infl_pm;
         if (s != ADMP_OK) return s;
         ctx->err.clear();
         return body();

@@ -301,7 +301,12 @@ hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t* g) {
     g_capture = nullptr;
     return *g ? hipSuccess : hipErrorInvalidValue;
 }
-hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t g, void*, void*, size_t) { *e = new emu_graph_exec{*g}; return hipSuccess; }
+// EMU_GRAPH_FAIL: no graph can be instantiated, as after a capture that another thread broke
+hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t g, void*, void*, size_t) {
+    if (getenv("EMU_GRAPH_FAIL")) return hipErrorUnknown;
+    *e = new emu_graph_exec{*g};
+    return hipSuccess;
+}
 hipError_t hipGraphLaunch(hipGraphExec_t e, hipStream_t) {
     for (auto& op : e->g.ops) op();
     return hipSuccess;

@@ -192,6 +192,14 @@ def test_solver_kinds_in_turn_on_one_context(emu_lib, case):
         assert x == y, (SOLVER_SEQUENCES[case], n)
 
 
+def test_failed_captures_run_eagerly(emu_lib):
+    """Phases and chunks whose captured graph cannot be instantiated run eagerly, from the host
+    state before the capture: the results are those of new contexts, bit by bit."""
+    a, b = (run(emu_lib, "solver_sequence", how, 1, extra_env=e)
+            for how, e in (("one", {"EMU_GRAPH_FAIL": "1"}), ("fresh", None)))
+    assert a == b
+
+
 def test_water_box_several_solver_blocks(emu_lib):
     """1,536 atoms: six solver blocks, the fused gather epilogue and a warm start."""
     r64 = run(emu_lib, "waters", "fp64", 512)
