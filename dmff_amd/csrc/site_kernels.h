@@ -810,7 +810,9 @@ __device__ inline double block_red(double v, double* sh) {
 // (pme.py:390-395) U -= g pol / DIELECTRIC.  Every block of the update reduces the same
 // maxima, so no launch or host round trip lies between test and update (2,970 sites, eleven
 // sweeps: 1,724 us per evaluation with the test on the host and four launches more, 1,227 so).
-// A converged frame keeps its U; tol < 0: no test.
+// A converged frame keeps its U: its maxima stay as they were, so the update's test repeats
+// itself.  The update does not ask for the frame's flag, which block 0 sets in the same launch:
+// wavefronts of a block could find it different.  tol < 0: no test.
 __global__ void __launch_bounds__(256)
 k_jacobi_grad(int N, double f1, const double* __restrict__ pol, const double* __restrict__ v,
               const double* __restrict__ real, const double* __restrict__ recip, const double* __restrict__ b,
@@ -842,14 +844,13 @@ k_jacobi(int N, int sweep, double tol, const double* __restrict__ pol, const dou
     __shared__ double sh[16];
     const int f = blockIdx.y;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (st[f].done) return;   // (also where block 0 has just set it: its test is every block's)
     double mx = 0;
     for (int k = threadIdx.x; k < (int)gridDim.x; k += blockDim.x) mx = fmax(mx, part[(size_t)f * gridDim.x + k]);
     mx = block_red<true>(mx, sh);
     const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
     if (lead) st[f].res = mx;
     if (mx < tol) {
-        if (lead) {
+        if (lead && !st[f].done) {
             st[f].iter = sweep;
             st[f].done = 1;
         }

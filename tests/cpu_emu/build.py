@@ -16,7 +16,11 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 REPO = os.path.dirname(os.path.dirname(HERE))
 
 
-def build(out_dir):
+FLAGS = ["-std=c++17", "-O2", "-fPIC", "-U_FORTIFY_SOURCE", "-D_FORTIFY_SOURCE=0", "-fno-strict-aliasing", "-w",
+         "-I" + HERE, "-x", "c++"]
+
+
+def _sources(out_dir):
     src = os.path.join(out_dir, "dmff_amd", "csrc")
     inc = os.path.join(out_dir, "include")
     os.makedirs(src, exist_ok=True)
@@ -33,9 +37,21 @@ def build(out_dir):
             with open(os.path.join(src, name), "w") as f:
                 f.write(text)
     shutil.copy(os.path.join(REPO, "include", "admp_hip.h"), inc)
+    return src
+
+
+def build(out_dir):
+    src = _sources(out_dir)
     lib = os.path.join(out_dir, "libadmp_emu.so")
-    cmd = ["g++", "-std=c++17", "-O2", "-fPIC", "-shared", "-U_FORTIFY_SOURCE", "-D_FORTIFY_SOURCE=0",
-           "-fno-strict-aliasing", "-w", "-I" + HERE, "-x", "c++", os.path.join(src, "admp_api.hip"),
-           os.path.join(HERE, "emu.cpp"), "-o", lib]
-    subprocess.run(cmd, check=True)
+    subprocess.run(["g++", "-shared", *FLAGS, os.path.join(src, "admp_api.hip"), os.path.join(HERE, "emu.cpp"), "-o", lib],
+                   check=True)
     return lib
+
+
+def build_kernel_cases(out_dir):
+    """A program that runs single kernels on chosen blocks (kernel_cases.cpp)."""
+    src = _sources(out_dir)
+    exe = os.path.join(out_dir, "kernel_cases")
+    subprocess.run(["g++", *FLAGS, "-I" + src, os.path.join(HERE, "kernel_cases.cpp"), os.path.join(HERE, "emu.cpp"), "-o",
+                    exe], check=True)
+    return exe

@@ -22,6 +22,7 @@ static const size_t STK = 128 * 1024;
 static std::vector<Fiber*> F;
 static jmp_buf sched_jb;
 Fiber* g_cur = nullptr;
+void (*g_after_wave)() = nullptr;
 static uint3e g_b, g_bd, g_gd;
 static const char* g_name = "";
 static size_t g_smem = 0;
@@ -237,7 +238,10 @@ void run_block(void (*entry)(void*), void* arg, unsigned bx, unsigned by, unsign
     }
     for (;;) {
         // each wavefront runs until all its fibres are at a barrier or done
-        for (unsigned w0 = 0; w0 < n; w0 += 64) run_wave(w0, std::min(n, w0 + 64), bx, by, bz);
+        for (unsigned w0 = 0; w0 < n; w0 += 64) {
+            run_wave(w0, std::min(n, w0 + 64), bx, by, bz);
+            if (g_after_wave) g_after_wave();
+        }
         unsigned done = 0;
         for (unsigned t = 0; t < n; ++t) done += F[t]->state == 3;
         if (done == n) break;

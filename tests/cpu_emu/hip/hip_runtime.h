@@ -44,6 +44,7 @@ inline double4 make_double4(double a, double b, double c, double d) { return dou
 namespace emu {
 struct Fiber;
 extern Fiber* g_cur;
+extern void (*g_after_wave)();   // called whenever a wavefront has come to a barrier or its end
 const uint3e& tidx();
 const uint3e& bidx();
 const uint3e& bdim();

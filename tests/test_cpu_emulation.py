@@ -40,6 +40,14 @@ def emu_lib(tmp_path_factory):
     return build(str(tmp_path_factory.mktemp("emu")))
 
 
+@pytest.fixture(scope="module")
+def kernel_cases(tmp_path_factory):
+    if shutil.which("g++") is None:
+        pytest.skip("g++ is needed to build the CPU emulation")
+    from tests.cpu_emu.build import build_kernel_cases
+    return build_kernel_cases(str(tmp_path_factory.mktemp("kernel_cases")))
+
+
 def run(lib, *args, timeout=900, extra_env=None):
     env = dict(os.environ, PYTHONPATH=REPO + os.pathsep + os.environ.get("PYTHONPATH", ""))
     env.update(extra_env or {})
@@ -198,6 +206,14 @@ def test_failed_captures_run_eagerly(emu_lib):
     a, b = (run(emu_lib, "solver_sequence", how, 1, extra_env=e)
             for how, e in (("one", {"EMU_GRAPH_FAIL": "1"}), ("fresh", None)))
     assert a == b
+
+
+@pytest.mark.parametrize("case", ["jacobi_flag"])
+def test_single_kernels(kernel_cases, case):
+    """jacobi_flag: a frame's converged flag, set by block 0 of the update while another block of
+    the launch runs, does not part that block's wavefronts."""
+    p = subprocess.run([kernel_cases, case], capture_output=True, text=True, timeout=300)
+    assert p.returncode == 0, p.stdout + p.stderr
 
 
 def test_water_box_several_solver_blocks(emu_lib):
