@@ -42,9 +42,31 @@ static int jacobi_flag() {
     return bad;
 }
 
+// k_cg_update, block 1 of 4, the same: the residual of parity 0 is below tol
+static int cg_flag() {
+    const int nb = 4, N = nb * PCG_BLOCK, n3 = 3 * N;
+    std::vector<double> pol(N, 1.0), x(n3, 0.0), r(2 * n3, 1e4), z(n3, 1.0), p(n3, 1.0), s(2 * n3, 1.0), w(n3, 1.0),
+        rec(N * MREC, 0.0), parts(nb + 4 * nb, 1.0);
+    const CgParts cp{parts.data(), nb, nb};
+    BoxInfo box{};
+    std::fill(cp.mx(0, 0), cp.mx(0, 0) + nb, 1e3);
+    int bad = 0;
+    for (int pass = 0; pass < 2; ++pass) {
+        g_st = PcgState{};
+        one_block(k_cg_update<double>, dim3(nb), dim3(PCG_BLOCK), 1, N, nb, 0, 1.0, (const BoxInfo*)&box, pol.data(), x.data(),
+                  r.data(), z.data(), p.data(), s.data(), w.data(), rec.data(), (double*)nullptr, (const int*)nullptr,
+                  (const double*)nullptr, cp, &g_st);
+        if (pass) for (double v : x) bad += v != 0.0;
+        std::fill(cp.mx(0, 0), cp.mx(0, 0) + nb, 0.1);
+        std::fill(x.begin(), x.end(), 0.0);
+        emu::g_after_wave = set_done;
+    }
+    return bad;
+}
+
 int main(int argc, char** argv) {
     const std::string c = argc > 1 ? argv[1] : "";
-    const int bad = c == "jacobi_flag" ? jacobi_flag() : -1;
+    const int bad = c == "jacobi_flag" ? jacobi_flag() : c == "cg_flag" ? cg_flag() : -1;
     printf("%s: %d wrong values\n", c.c_str(), bad);
     return bad != 0;
 }
