@@ -380,6 +380,9 @@ k_nbr_build(int N, int cap, const double4* __restrict__ pos, const BoxInfo* __re
             const double* Bi = bm.Binv + d;
             double sd = pi_.x * Bi[0] + pi_.y * Bi[3] + pi_.z * Bi[6];
             sd = (sd - floor(sd)) * cg.nc[d] - cc[d];                       // place in the own cell, 0..1
+            // (k_cell_assign's rounding may have found a site on the periodic face on the other side)
+            if (sd > 1.5) sd -= cg.nc[d];
+            if (sd < -0.5) sd += cg.nc[d];
             const int n = cg.nc[d], off = (at[d] - cc[d] + n) % n;
             const double up = off == 1 ? 1.0 - sd : 1e30, down = off == n - 1 ? sd : 1e30;
             const double w = 1.0 / (n * sqrt(Bi[0] * Bi[0] + Bi[3] * Bi[3] + Bi[6] * Bi[6]));   // slab width

@@ -64,9 +64,40 @@ static int cg_flag() {
     return bad;
 }
 
+// k_nbr_build with a site on the periodic face whose stored cell and recomputed place lie on
+// opposite sides of it, as two kernels' roundings may have it: its neighbours on either side stay.
+// (lo: the site at 0+, stored in the last cell; else at the box's end, stored in the first.)
+static int nbr_face(bool lo, int nc) {
+    const double rc = 4.0, L = nc * rc * 1.004;
+    const int N = 3, cap = 8;
+    const double x0 = lo ? 1e-17 : L * (1.0 - 1e-16);
+    // neighbours 0.5 beyond either side of the face, in the last and the first cell
+    const double4 pos[N] = {make_double4(x0, 1, 1, 0), make_double4(L - 0.5, 1, 1, 0), make_double4(0.5, 1, 1, 0)};
+    BoxInfo box{};
+    for (int d = 0; d < 3; ++d) { box.B[4 * d] = L; box.Binv[4 * d] = 1.0 / L; }
+    const CellGrid cg{{nc, 1, 1}, nc};
+    const int cell[N] = {lo ? nc - 1 : 0, nc - 1, 0};
+    std::vector<int> start(nc + 1, 0);
+    for (int c : cell) ++start[c + 1];
+    for (int c = 0; c < nc; ++c) start[c + 1] += start[c];
+    std::vector<int> fill(start);
+    double4 spos[N];
+    for (int i = 0; i < N; ++i) { spos[fill[cell[i]]] = pos[i]; spos[fill[cell[i]]++].w = i; }
+    const int xoff[N + 1] = {0, 0, 0, 0}, xent[1] = {0};
+    int nbr[N * cap], ncnt[N], nhalf[N], maxcnt = 0;
+    one_block(k_nbr_build, dim3(1), dim3(256), 0, N, cap, pos, (const BoxInfo*)&box, cg, rc * rc, cell, (const int*)start.data(),
+              (const double4*)spos, xoff, xent, nbr, ncnt, nhalf, &maxcnt);
+    return (ncnt[0] != 2) + (ncnt[1] != 2) + (ncnt[2] != 2);
+}
+static int nbr_faces() {
+    int bad = 0;
+    for (int nc : {2, 3, 4, 7}) bad += nbr_face(true, nc) + nbr_face(false, nc);
+    return bad;
+}
+
 int main(int argc, char** argv) {
     const std::string c = argc > 1 ? argv[1] : "";
-    const int bad = c == "jacobi_flag" ? jacobi_flag() : c == "cg_flag" ? cg_flag() : -1;
+    const int bad = c == "jacobi_flag" ? jacobi_flag() : c == "cg_flag" ? cg_flag() : c == "nbr_faces" ? nbr_faces() : -1;
     printf("%s: %d wrong values\n", c.c_str(), bad);
     return bad != 0;
 }

@@ -208,10 +208,11 @@ def test_failed_captures_run_eagerly(emu_lib):
     assert a == b
 
 
-@pytest.mark.parametrize("case", ["jacobi_flag", "cg_flag"])
+@pytest.mark.parametrize("case", ["jacobi_flag", "cg_flag", "nbr_faces"])
 def test_single_kernels(kernel_cases, case):
     """jacobi_flag, cg_flag: a frame's converged flag, set by block 0 of the update while another block of
-    the launch runs, does not part that block's wavefronts."""
+    the launch runs, does not part that block's wavefronts.  nbr_faces: a site on the periodic
+    face keeps its neighbours where two kernels round its place to opposite sides."""
     p = subprocess.run([kernel_cases, case], capture_output=True, text=True, timeout=300)
     assert p.returncode == 0, p.stdout + p.stderr
 
