@@ -1028,10 +1028,7 @@ __global__ void __launch_bounds__(PCG_BLOCK) k_cg_update(int N, int nwu, int cur
     // reductions that give them, so the wave waits for memory once, not four
     // times in a row (state, partial sums, site vectors, partner vectors).
     const double gp = st[f].gam[nx], ap = st[f].alp[nx];
-    // The flag of a frame that converged before.  Without PME no product tests the residual, and
-    // block 0 sets it below: one thread reads it for the block (at the barriers of the totals).
-    __shared__ int done;
-    if (threadIdx.x == 0) done = st[f].done;
+    const int done = st[f].done;
     const size_t a = (size_t)f * N + (i < N ? i : 0);
     double zv[3] = {0, 0, 0}, pv0[3] = {0, 0, 0}, wv[3] = {0, 0, 0}, sv0[3] = {0, 0, 0}, rv0[3] = {0, 0, 0};
     double wj[3][3] = {}, sj[3][3] = {}, rj0[3][3] = {};
@@ -1060,9 +1057,14 @@ __global__ void __launch_bounds__(PCG_BLOCK) k_cg_update(int N, int nwu, int cur
                 }
             }
     }
+    // The flag of a frame that converged before.  Without PME no product tests the residual, and
+    // block 0 sets the flag below: the block takes what one of its threads read (at the barriers
+    // of the totals).
+    __shared__ int block_done;
+    if (threadIdx.x == 0) block_done = done;
     double res, gamma, delta;
     parts_total_cg(parts.mx(f, cur), parts.rz(f, cur), parts.nb, parts.zw(f), nwu, sh, res, gamma, delta);
-    if (done) return;
+    if (block_done) return;
     const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
     if (res < tol) {
         if (lead) {
