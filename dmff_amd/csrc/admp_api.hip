@@ -740,13 +740,16 @@ extern "C" admp_status admp_ctx_create(const admp_config* cfg, admp_ctx** out) {
         ALLOC(ctx->d_gcfill, Gmax * ctx->F);
         ALLOC(ctx->d_gcstart, (Gmax + 1) * ctx->F);
         // brick lists for the radix path (FP32 passes, grids beyond the matrix-core
-        // passes), tile lists for the matrix-core passes
+        // passes), tile lists for the matrix-core passes: those of FP64 arithmetic, which a
+        // mixed context has in its solves alone (the tile lists are 384 bytes per site: 0.3 GB
+        // for 64 frames of 12,288 sites)
+        auto runs_mm = [&](const Grid* gg) { return gg->mm && (!mixed || (gg == &ctx->eg && c.lpol)); };
         size_t nbrmax = 0, ntmax = 0;
         for (const Grid* gg : {&ctx->eg, &ctx->dg})
             if (gg->G) {
                 const size_t nxy = (size_t)((gg->K[0] + BRX - 1) / BRX) * ((gg->K[1] + BRY - 1) / BRY);
                 if (mixed || !gg->mm) nbrmax = std::max(nbrmax, nxy * ((gg->K[2] + BRZ - 1) / BRZ));
-                if (gg->mm) {
+                if (runs_mm(gg)) {
                     ntmax = std::max(ntmax, nxy * mm_nseg(gg->K[2]));
                     ctx->gz_tiles = std::max(ctx->gz_tiles, (int)nxy);
                 }
@@ -765,7 +768,7 @@ extern "C" admp_status admp_ctx_create(const admp_config* cfg, admp_ctx** out) {
         }
         if (ctx->eg.G)
             ALLOC(ctx->d_infl, (size_t)ctx->eg.K[0] * ctx->eg.K[1] * (ctx->eg.K[2] / 2 + 1) * ctx->F);
-        if (ctx->dg.mm)
+        if (runs_mm(&ctx->dg))
             ALLOC(ctx->d_dinfl, 2 * (size_t)ctx->dg.K[0] * ctx->dg.K[1] * (ctx->dg.K[2] / 2 + 1) * ctx->F);
     }
     ALLOC(ctx->d_wd, NF * 3);

@@ -410,6 +410,13 @@ def cfg3s(precision):
             "e_pol": info["e_pol"], "n_iter": info["n_iter"][0], "pos": _lst(g["pos"][0])}
 
 
+def memory(precision):
+    """Device memory of a context that runs FP32 passes alone: not polarisable, dispersion."""
+    from dmff_amd.admp.engine import Engine
+    eng = Engine(300, 2, False, True, 0.4, (18, 19, 17), 6.0, dK=(20, 21, 16), disp_kappa=0.4, precision=precision)
+    return eng.memory_bytes()
+
+
 def qeq(variant):
     """ADMPQeqForce on the small charge-equilibration case: periodic (damp_mod 3,
     slab correction) or not (damp_mod 2): energy, charges, and gradients with
@@ -431,7 +438,7 @@ def qeq(variant):
             "pos": _lst(g[0]), "box": _lst(g[1]), "chi": _lst(g[2]), "J": _lst(g[3]), "eta": _lst(g[4])}
 
 
-CASES = {"qeq": qeq, "cfg3s": cfg3s, "axis_types": axis_types, "triclinic": triclinic, "coul": coul, "esp": esp, "generators": generators, "pairwise": pairwise, "bad_geometry": bad_geometry, "type_reduce": type_reduce, "small_box": small_box, "frames": frames, "disp_slater": disp_slater, "neighbors": neighbors}
+CASES = {"qeq": qeq, "memory": memory, "cfg3s": cfg3s, "axis_types": axis_types, "triclinic": triclinic, "coul": coul, "esp": esp, "generators": generators, "pairwise": pairwise, "bad_geometry": bad_geometry, "type_reduce": type_reduce, "small_box": small_box, "frames": frames, "disp_slater": disp_slater, "neighbors": neighbors}
 
 if __name__ == "__main__":
     lib, case = sys.argv[1], sys.argv[2]

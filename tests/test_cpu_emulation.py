@@ -208,6 +208,13 @@ def test_failed_captures_run_eagerly(emu_lib):
     assert a == b
 
 
+def test_fp32_passes_hold_no_matrix_core_buffers(emu_lib):
+    """A mixed context that runs FP32 passes alone holds what it holds where the matrix-core
+    passes are off: no tile lists, no tables of theirs."""
+    a, b = (run(emu_lib, "memory", "mixed", extra_env=e) for e in (None, {"ADMP_SPREAD": "cw"}))
+    assert a == b
+
+
 @pytest.mark.parametrize("case", ["jacobi_flag", "cg_flag", "nbr_faces"])
 def test_single_kernels(kernel_cases, case):
     """jacobi_flag, cg_flag: a frame's converged flag, set by block 0 of the update while another block of
