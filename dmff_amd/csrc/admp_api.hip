@@ -2318,6 +2318,14 @@ static PairParams make_pp(const double* mS, const double* pS, const double* dS, 
     return pp;
 }
 
+// The FP64 final pass without induced dipoles leaves registers to the reciprocal chain beside it:
+// for one frame, and for batches up to 32,768 sites, where the chain's launches are a large part
+// of the evaluation (12,288 sites, 50^3: 382 us with the register file full, 331 so; 98,304 sites
+// with 80 neighbours each, 80^3: 782 and 722; 8 frames of 3,000, 32^3: 379 and 352).  In larger
+// batches the pair pass itself counts for more (64 frames of 3,000: 1577 and 1630; 8 of 12,288:
+// 1259 and 1292).
+static bool real_final_room(const admp_ctx* ctx) { return ctx->F == 1 || (long)ctx->N * ctx->F <= 32768; }
+
 template <class R>
 static admp_status compute_impl(admp_ctx* ctx, const double* Q_local, const double* pol, const double* thole,
                                 const PairParams& pp, double* U_inout, const admp_solver_opts* opts, int want_grad,
@@ -2353,14 +2361,15 @@ static admp_status compute_impl(admp_ctx* ctx, const double* Q_local, const doub
         HIPCHK(hipEventRecord(ctx->ev_fork, st));
         HIPCHK(hipStreamWaitEvent(sr, ctx->ev_fork, 0));
     }
-    if (lpol)
-        { ProfScope ps_(ctx, 0, sr); hipLaunchKernelGGL((k_real_final<R, true>), pgrid, dim3(PAIR_BLOCK), 0, sr, N, ctx->cap, ctx->d_pos, ctx->d_box,
-                           site, ctx->d_nbr, ctx->d_ncnt, pp, ctx->d_e_atom, ctx->d_gpos, ctx->d_gq, ctx->d_vir_atom,
-                           ctx->d_gpol, ctx->d_gth); }
-    else
-        { ProfScope ps_(ctx, 0, sr); hipLaunchKernelGGL((k_real_final<R, false>), pgrid, dim3(PAIR_BLOCK), 0, sr, N, ctx->cap, ctx->d_pos, ctx->d_box,
-                           site, ctx->d_nbr, ctx->d_ncnt, pp, ctx->d_e_atom, ctx->d_gpos, ctx->d_gq, ctx->d_vir_atom,
-                           ctx->d_gpol, ctx->d_gth); }
+    {
+        ProfScope ps_(ctx, 0, sr);
+        auto kernel = lpol ? k_real_final<R, true, 8> : k_real_final<R, false, 8>;
+        if constexpr (sizeof(R) == 8)
+            if (!lpol && lpme && real_final_room(ctx)) kernel = k_real_final<R, false, 2>;
+        hipLaunchKernelGGL(kernel, pgrid, dim3(PAIR_BLOCK), 0, sr, N, ctx->cap, ctx->d_pos, ctx->d_box, site, ctx->d_nbr,
+                           ctx->d_ncnt, pp, ctx->d_e_atom, ctx->d_gpos, ctx->d_gq, ctx->d_vir_atom, ctx->d_gpol,
+                           ctx->d_gth);
+    }
     HIPCHK(hipGetLastError());
     if (!lpol) {
         HIPCHK(hipMemsetAsync(ctx->d_gpol, 0, NF * sizeof(double), sr));

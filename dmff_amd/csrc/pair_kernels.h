@@ -383,10 +383,13 @@ __device__ __forceinline__ void real_final64(int N, int cap, const double4* __re
 }
 
 // ---------------------------------------------------------------------------
-// Final pass: energy and every gradient, U held fixed.
+// Final pass: energy and every gradient, U held fixed.  MAXW: most wavefronts per SIMD.  The
+// FP64 pass without induced dipoles has 162 registers: three wavefronts fill a SIMD's register
+// file, and the reciprocal chain of launches beside it waits until they end.  With two, the
+// chain's small launches run beside the pass (real_final_room in admp_api.hip).
 // ---------------------------------------------------------------------------
-template <class R, bool LPOL>
-__global__ void __launch_bounds__(PAIR_BLOCK, sizeof(R) == 8 ? 2 : 1)
+template <class R, bool LPOL, int MAXW>
+__global__ void __launch_bounds__(PAIR_BLOCK) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 2 : 1, MAXW)))
 k_real_final(int N, int cap, const double4* __restrict__ pos, const BoxInfo* __restrict__ boxes,
              const R* __restrict__ site, const int* __restrict__ nbr, const int* __restrict__ ncnt,
              PairParams pp, double* __restrict__ e_atom, double* __restrict__ g_pos,

@@ -605,6 +605,30 @@ def test_matrix_core_grids(K):
     assert errs.pop("E") < 1e-9 and max(errs.values()) < 1e-7
 
 
+@pytest.mark.parametrize("n_frames", [248, 249])
+def test_final_pass_of_batches_without_dipoles(n_frames):
+    """248 frames of 132 sites (32,736) leave registers to the reciprocal chain, 249 fill the register
+    file: both are the single frames (same terms in the same order: 1e-13 relative)."""
+    from dmff_amd.admp.engine import Engine
+    s, pos, box = _small_waters()
+    rng = np.random.default_rng(31)
+    P = np.stack([pos + rng.normal(0, 0.02, pos.shape) for _ in range(n_frames)])
+
+    def evaluate(Pf):
+        n = len(Pf)
+        eng = Engine(len(pos), 2, False, True, 0.4, (18, 19, 17), 6.0, n_frames=n, device=DEV)
+        eng.set_topology(s.axis_types, s.axis_idx, s.bonded)
+        eng.build_neighbors(Pf, np.stack([box] * n))
+        E, g, U, info = eng.compute(Pf, np.stack([box] * n), s.pme.Q_local[s.map_atomtype], mScales=s.pme.mScales)
+        return [x.cpu().numpy() for x in (E, g["pos"], g["box"], g["Q"])]
+
+    batch = evaluate(P)
+    assert len(pos) == 132
+    for k in (0, n_frames - 1):
+        for a, b in zip(batch, evaluate(P[k:k + 1])):
+            assert rel_rms(a[k], b[0]) < 1e-13
+
+
 @pytest.mark.parametrize("case", range(len(SOLVER_SEQUENCES)))
 def test_solver_kinds_in_turn_on_one_context(case):
     """Calls with different solvers on one mixed context, whose phases are captured and replayed:
