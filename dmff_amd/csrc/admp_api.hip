@@ -480,6 +480,38 @@ static int spread_wpt(int K0, int K1, int K2, int F, int lm) {
     return w;
 }
 
+// Grids whose FP64 passes stay on the radix path.  The dense transforms cost K^2 per line: past
+// 63 points (a third row tile), past the plane that fits the LDS (97^2), and past a z axis of 96
+// (the spread and the gather take a CU's LDS for one workgroup) they lose to radix passes whose
+// stages are short, i.e. axes of which no prime factor is above 5 (or 7 times a power of two);
+// with longer stages they win everywhere up to MM_KMAX (12,288 sites: 88 points 3.87 ms radix,
+// 2.05 here; 91: 5.15 and 2.32; 127: 785 and 13).  ms per evaluation, radix / here:
+//   solves, one frame of 12,288 sites: 80^3 2.32 / 2.03, 90^3 2.61 / 2.33, 80 x 80 x 120
+//     2.67 / 2.35, 96^3 2.88 / 3.02, 120^3 3.48 / 3.99, 128^3 4.33 / 5.68, 64 x 128 x 128
+//     3.01 / 3.30; of 98,304: 96^3 19.8 / 21.2, 128^3 24.5 / 27.1
+//   solves, eight frames: 80^3 7.38 / 7.43, 90^3 9.14 / 8.72, 100^3 11.7 / 13.6, 128^3 21.6 /
+//     36.5; 60 x 60 x 120 7.06 / 7.72, 50 x 50 x 128 6.04 / 7.95
+//   one evaluation without dipoles, 12,288 sites: 64^3 0.304 / 0.288, 75^3 0.322 / 0.354, 96^3
+//     0.402 / 0.438; of 98,304 level (100^3 1.38 / 1.33); eight frames: 90^3 1.36 / 1.30, 100^3
+//     1.58 / 2.01
+//   dispersion, 8,580 sites: 60^3 0.615 / 0.574, 75^3 0.673 / 0.713, 96^3 0.80 / 0.95; eight
+//     frames: 60^3 1.06 / 0.93, 64^3 1.11 / 1.17, 96^3 2.09 / 2.88
+static bool radix_faster(const admp_ctx* ctx, const Grid& g) {
+    for (int K : g.K) {
+        int odd = K;
+        while (odd % 2 == 0) odd /= 2;
+        if (odd == 7) continue;
+        for (int p : {3, 5})
+            while (odd % p == 0) odd /= p;
+        if (odd > 1) return false;
+    }
+    auto past = [&](long k) { return g.G > (size_t)(k * k * k); };
+    const bool batch = ctx->F > 1;
+    if (&g == &ctx->dg) return past(batch ? 60 : 64);
+    if (!ctx->cfg.lpol) return batch ? past(90) : past(64) && ctx->N <= 65536;
+    return batch ? past(90) || (past(64) && g.K[2] > 96) : past(82) && g.K[0] * g.K[1] > 90 * 90;
+}
+
 static admp_status setup_grid(admp_ctx* ctx, Grid& g, int K0, int K1, int K2, bool mixed) {
     g.K[0] = K0; g.K[1] = K1; g.K[2] = K2;
     g.G = (size_t)K0 * K1 * K2;
@@ -520,10 +552,10 @@ static admp_status setup_grid(admp_ctx* ctx, Grid& g, int K0, int K1, int K2, bo
     // tables in LDS.  It is used up to PLANE_LDS_MAX bytes (two blocks per CU;
     // up to 50^2 in FP64, 71^2 in FP32); larger planes take the line passes.
     const char* env = std::getenv("ADMP_FFT_PLANE");
-    // The FP64 passes run on the matrix cores up to MM_KMAX points per axis, with the
-    // plane in LDS where it fits one workgroup per CU.
+    // The FP64 passes run on the matrix cores up to MM_KMAX points per axis, but where the radix
+    // passes are faster, with the plane in LDS where it fits one workgroup per CU.
     g.mm = K0 <= MM_KMAX && K1 <= MM_KMAX && K2 <= MM_KMAX && K0 >= BRX + 5 && K1 >= BRY + 5 && K2 >= BRZ + 5 &&
-           !spread_forced() && mm_kernels_ready();
+           !spread_forced() && !radix_faster(ctx, g) && mm_kernels_ready();
     g.mm_plane = g.mm && plane_mm_lds(K0, K1) <= MM_PLANE_LDS && !(env && env[0] == '0');
     const bool allow = !(env && env[0] == '0') && K0 >= BRX + 5 && K1 >= BRY + 5 && K2 >= BRZ + 5;
     for (int w = 0; w < 2; ++w) {

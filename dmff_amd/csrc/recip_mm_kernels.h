@@ -7,11 +7,12 @@
 // e_n = x_n + x_{K-n} and o_n = x_n - x_{K-n} (n <= K / 2), so that
 //   C_k = sum_n e_n cos(2 pi k n / K),   S_k = sum_n o_n sin(2 pi k n / K)
 // give frequencies k and K - k at once: H = K / 2 + 1 rows and columns, a quarter of
-// the products of the full matrix.  At the grid sizes of the Ewald rule (13..100
-// points) this costs less than the LDS passes, barriers and index arithmetic of a
-// mixed-radix transform, and it does not depend on the factors of K: the radix
-// passes of recip2_kernels.h fall back to a direct sum by one thread per line where
-// K is prime.  The FP32 passes of the mixed path keep the radix transforms.
+// the products of the full matrix.  Up to about 64 points this costs less than the LDS
+// passes, barriers and index arithmetic of a mixed-radix transform, up to about 90 as
+// much, and it does not depend on the factors of K: the radix passes of
+// recip2_kernels.h fall back to a direct sum by one thread per line where K is prime.
+// Large grids of small factors stay there (radix_faster in admp_api.hip), and so do the
+// FP32 passes of the mixed path.
 //
 // Measured per product, radix passes -> these: 12,288 sites on 50 x 50 x 50 (15 of them per
 // solve): spread 14.6 + r2c 7.5 -> 15.6, plane 18.0 -> 21.6, c2r 6.5 + gather 8.1 -> 12.0 us;

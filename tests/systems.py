@@ -300,6 +300,8 @@ def library_pme(pos, box, axis_types, axis_idx, bonded, Q, pol, thole, scales, r
 # 63 | 64 points are one row tile | two and two | three; odd and even, primes, the shortest and
 # the longest axes, axes of a tile that is only part full, and planes past the LDS (y and x
 # lines in passes of their own)
+# grids of small factors on either side of the line past which they stay on the radix path
+RADIX_GRIDS = [(90, 90, 90), (96, 90, 90), (54, 50, 96), (54, 50, 100)]
 MATRIX_GRIDS = [(9, 10, 11), (31, 32, 16), (17, 33, 31), (12, 63, 64), (13, 9, 128), (97, 101, 10), (128, 127, 9)]
 
 

@@ -12,7 +12,7 @@ import pytest
 import torch
 
 from oracle import admp_oracle as O
-from tests.systems import (MATRIX_GRIDS, SOLVER_SEQUENCES, load_system, polar_grid, polar_grid_oracle, reference_pairs,
+from tests.systems import (MATRIX_GRIDS, RADIX_GRIDS, SOLVER_SEQUENCES, load_system, polar_grid, polar_grid_oracle, reference_pairs,
                            small_water_box as _small_waters, solver_sequence)
 
 pytestmark = pytest.mark.gpu
@@ -600,6 +600,16 @@ def test_matrix_core_grids(K):
     9 x 10 x 11, by either path; below 1e-12 from 16 points on)."""
     a, o = polar_grid(K, DEV), polar_grid_oracle(K)
     del o["box"]
+    errs = {k: rel_rms(a[k][0], o[k]) for k in o}
+    print(f"K={K}: {errs}", flush=True)
+    assert errs.pop("E") < 1e-9 and max(errs.values()) < 1e-7
+
+
+@pytest.mark.parametrize("K", RADIX_GRIDS)
+def test_grids_beside_the_radix_line(K):
+    """Two frames on either side of the lines past which grids of small factors stay on the radix
+    path: the oracle on the same grid, to the tolerances above, box included (no axis below 16)."""
+    a, o = polar_grid(K, DEV), polar_grid_oracle(K)
     errs = {k: rel_rms(a[k][0], o[k]) for k in o}
     print(f"K={K}: {errs}", flush=True)
     assert errs.pop("E") < 1e-9 and max(errs.values()) < 1e-7
