@@ -2879,9 +2879,19 @@ namespace {
 
 constexpr int NA_BLOCK = 512;
 constexpr int NA_MAXBLK = 1024;
-constexpr int NA_CHUNK = 2048;                             // pairs whose gradients meet in one LDS table
+constexpr int NA_CHUNK = 2048;                             // most pairs whose gradients meet in one LDS table
 constexpr int NA_SLOTS = 1024;                             // sites of the table
 constexpr int NA_PROBES = 8;
+// Pairs per chunk: as few as give every CU one (at least 256), since a chunk's rows take turns and
+// share a table that a list in no order overfills.  Sorted / shuffled lists of 20,800 pairs of
+// 3,000 sites, with chunks of 2048: 38 / 51 us; 256: 20 / 20; an atomic per value: 92 / 39.  Long
+// sorted lists gain from the longer runs of 2048 (332,000 pairs: 43 us; 1024: 51; 512: 57), long
+// shuffled ones would lose less with short chunks (148, 126, 99; an atomic per value: 407).
+__host__ __device__ inline int na_chunk(int64_t np) {
+    int c = 256;
+    while (c < NA_CHUNK && np > 256 * (int64_t)c) c *= 2;
+    return c;
+}
 constexpr int NA_BOX_DOUBLES = 64;                         // BoxInfo + the flag word
 constexpr int NA_SCRATCH_DOUBLES = NA_BOX_DOUBLES + NA_MAXBLK * 10;  // 82,432 bytes
 static_assert(sizeof(BoxInfo) + sizeof(int) <= NA_BOX_DOUBLES * sizeof(double), "box record");
@@ -2972,7 +2982,8 @@ k_na_pairs(int64_t np, int N, const I* __restrict__ pairs, const double* __restr
         }
         return nullptr;
     };
-    const int64_t nch = (np + NA_CHUNK - 1) / NA_CHUNK;
+    const int chunk = na_chunk(np);
+    const int64_t nch = (np + chunk - 1) / chunk;
     for (int64_t c = blockIdx.x; c < nch; c += gridDim.x) {
         if (want_grad) {
             __syncthreads();   // the table of the chunk before has gone out
@@ -2980,8 +2991,8 @@ k_na_pairs(int64_t np, int N, const I* __restrict__ pairs, const double* __restr
             for (int t = threadIdx.x; t < NA_SLOTS; t += NA_BLOCK) key[t] = -1;
             __syncthreads();
         }
-        const int64_t r1 = min(np, (c + 1) * NA_CHUNK);
-        for (int64_t r = c * NA_CHUNK + threadIdx.x; r < r1; r += NA_BLOCK) {
+        const int64_t r1 = min(np, (c + 1) * chunk);
+        for (int64_t r = c * chunk + threadIdx.x; r < r1; r += NA_BLOCK) {
             const int64_t i = (int64_t)pairs[r * 3], j = (int64_t)pairs[r * 3 + 1];
             if (!(i >= 0 && i < j && j < N)) continue;
             const int64_t nb64 = (int64_t)pairs[r * 3 + 2];
@@ -3104,7 +3115,7 @@ extern "C" admp_status admp_pairwise_compute_noalloc(int32_t kind, int32_t preci
     const PairParams pp = make_pp(mScales, nullptr, nullptr, n_scales, 0.0);
     double* gp = want_grad ? dpos : nullptr;
     double* gq = want_grad ? dprm : nullptr;
-    const int64_t want_blocks = (n_pairs + NA_CHUNK - 1) / NA_CHUNK;
+    const int64_t want_blocks = (n_pairs + na_chunk(n_pairs) - 1) / na_chunk(n_pairs);
     const int nb = (int)std::max<int64_t>(1, std::min<int64_t>(want_blocks, NA_MAXBLK));
     const size_t nz = (size_t)n_atoms * std::max(3, (int)n_prm);
     hipLaunchKernelGGL(k_na_prep, dim3((unsigned)std::min<size_t>(nblk(nz, 256), 1024)), dim3(256), 0, st, n_atoms,

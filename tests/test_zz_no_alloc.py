@@ -91,6 +91,31 @@ def test_noalloc_chunks_and_full_site_table(order, n_pairs):
     assert max(errs) < 1e-12
 
 
+@pytest.mark.parametrize("order", ["sorted", "shuffled"])
+@pytest.mark.parametrize("n_pairs", [255, 256, 257, 65536, 65537, 131073, 262144, 262145, None])
+def test_noalloc_chunk_lengths(order, n_pairs):
+    """The lattice with pairs inside 12 A: list lengths at which a chunk's length doubles (256 to
+    2048 pairs); the longest shuffled list fills the table.  Tolerance as above."""
+    rng = np.random.default_rng(7)
+    g = np.stack(np.meshgrid(*[np.arange(12)] * 3, indexing="ij"), -1).reshape(-1, 3) * 2.5
+    pos, box = g + rng.uniform(-0.4, 0.4, g.shape), np.eye(3) * 30.0
+    d = pos[:, None] - pos[None]
+    d -= np.round(d / 30.0) * 30.0
+    i, j = np.nonzero(np.triu((d ** 2).sum(-1) < 144.0, 1))
+    pairs = np.stack([i, j, np.zeros_like(i)], 1)
+    assert len(pairs) > 262145
+    if order == "shuffled":
+        pairs = pairs[rng.permutation(len(pairs))]
+    pairs = pairs[:n_pairs]
+    prm = rng.uniform(2.0, 4.0, (len(pos), 4))
+    m = np.array([0.0, 0.0, 0.0, 1.0, 1.0, 1.0])
+    ref = _with_context(2, "fp64", pos, box, pairs, m, prm)
+    got = _noalloc(2, "fp64", pos, box, pairs, m, prm)
+    errs = [abs(got[0] - ref[0]) / abs(ref[0])] + [_rel(got[k], ref[k]) for k in (1, 2, 3)]
+    print(f"{order} {len(pairs)} pairs: {errs}", flush=True)
+    assert max(errs) < 1e-12
+
+
 @pytest.mark.parametrize("prec", ["fp64", "mixed"])
 @pytest.mark.parametrize("kind", [1, 2, 3, 4])
 def test_noalloc_equals_context_entry_point_twice(kind, prec):
