@@ -467,16 +467,15 @@ static int spread_forced() {
     return v;
 }
 
-// wavefronts sharing a z segment's candidates in k_spread_z
+// wavefronts sharing a z segment's candidates in k_spread_z: up to 8 per CU in all
 static int spread_wpt(int K0, int K1, int K2, int F, int lm) {
     const int nseg = mm_nseg(K2);
     const long tiles = (long)((K0 + MM_TX - 1) / MM_TX) * ((K1 + MM_TY - 1) / MM_TY) * F;
-    
     auto lds = [&](int n) {
         return lm == 0 ? spread_mm_lds<0>(K2, n) : lm == 1 ? spread_mm_lds<1>(K2, n) : spread_mm_lds<2>(K2, n);
     };
     int w = 1;
-    while (w < 4 && 2 * w * nseg <= 16 && tiles * nseg * w < 2048 && lds(2 * w) <= MM_LDS_MAX) w *= 2;
+    while (w < 4 && 2 * w * nseg <= 16 && tiles * nseg * w < 8 * N_CU && lds(2 * w) <= MM_LDS_MAX) w *= 2;
     return w;
 }
 
@@ -1771,13 +1770,16 @@ static admp_status pcg_apply(admp_ctx* ctx, const double* pol, double f1, int cu
     const bool fused = ctx->cfg.lpme && !small_grid(ctx->eg);
     // With few frames the plane pass fills only K2/2+1 workgroups per frame: the
     // real-space product then runs inside that launch (k_plane_matvec) instead of
-    // on the side stream, which saves the fork and the join of every iteration, as
-    // long as the CUs without a plane hold its lanes at once (98,304 sites beside 41
-    // planes of 80 x 80 are 3.6 rounds of them: 490 us per iteration in one launch
-    // against 460 on the side stream).
+    // on the side stream, which saves the fork and the join of every iteration, as long
+    // as the CUs without a plane hold its lanes in one round, were each to hold CU_LANES
+    // (its workgroups share the planes' LDS size, so beside planes above 64 x 64 they hold
+    // fewer).  That is about where the two meet: side stream / one launch, ms per
+    // evaluation, 18,000, 24,600 and 36,000 sites: 50^3 5.19 / 5.15, 8.59 / 8.95, 3.66 /
+    // 4.05; 64^3 5.83 / 5.53, 9.40 / 9.51, 4.31 / 4.84; 80^3 8.12 / 7.25, 13.8 / 12.3,
+    // 5.27 / 5.03; 49,000 sites on 80^3 12.4 / 13.1.
     const int np = (ctx->eg.K[2] / 2 + 1) * F;
     const bool plane = sizeof(R) == 8 && use_mm(ctx, ctx->eg) ? ctx->eg.mm_plane : ctx->eg.plane[sizeof(R) == 8 ? 1 : 0];
-    const bool with_plane = fused && plane && np <= 128 && (long)N * F * TPA <= 2048L * (256 - np);
+    const bool with_plane = fused && plane && np <= N_CU / 2 && (long)N * F * TPA <= (long)CU_LANES * (N_CU - np);
     // Otherwise it runs on the side stream, beside the reciprocal chain, and is launched once
     // the chain's spread is: launched before it, its workgroups hold every CU and the chain,
     // the longer of the two paths, waits (98,304 sites: 12.5 ms per evaluation against 11.9).

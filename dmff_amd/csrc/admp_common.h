@@ -37,6 +37,8 @@ template <class R> struct Cplx { R x, y; };
 // range: physical block p runs logical item (p % 8) * ceil(n / 8) + p / 8.  The
 // grid is launched with 8 * ceil(n / 8) blocks; logical items >= n return.
 constexpr int N_XCD = 8;
+constexpr int N_CU = 256;               // compute units, which the launch rules reckon with
+constexpr int CU_LANES = 2048;          // most resident lanes of one (32 wavefronts)
 __host__ __device__ inline int xcd_blocks(int n) { return ((n + N_XCD - 1) / N_XCD) * N_XCD; }
 __device__ inline int xcd_item(int p, int n) { return (p % N_XCD) * ((n + N_XCD - 1) / N_XCD) + p / N_XCD; }
 

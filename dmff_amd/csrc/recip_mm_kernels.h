@@ -48,7 +48,7 @@ __device__ __forceinline__ void wave_lds_fence() {
 // converged flag, which saves a load's latency; in one of several rounds of workgroups the
 // others cover that, and a converged frame's workgroups leave before they load anything
 // (64 converged frames of 169 tiles: 170 us against 7 for the gather).
-__device__ __forceinline__ bool early_exit() { return gridDim.x * gridDim.y > 1024; }
+__device__ __forceinline__ bool early_exit() { return gridDim.x * gridDim.y > 4 * N_CU; }
 
 // largest axis of the dense transforms: the products grow as K^2 per line
 constexpr int MM_KMAX = 128;
@@ -728,7 +728,7 @@ constexpr int GZ_THREADS = 64 * GZ_CT * 2;           // 12 wavefronts, 96 sites 
 // one tile's loads run beside another's products.  With 12 / 8 / 4 wavefronts: 44 / 40 / 49 us
 // for 400 tiles (98304 sites, 80 x 80 x 80), 436 / 309 / 293 us for 10816 (64 frames of 12288
 // sites, 50 x 50 x 50), and 3470 / 1156 / 700 us for the latter's final pass beside the pair kernel.
-__host__ inline int gather_z_threads(int items) { return items <= 256 ? GZ_THREADS : items <= 1024 ? 512 : 256; }
+__host__ inline int gather_z_threads(int items) { return items <= N_CU ? GZ_THREADS : items <= 4 * N_CU ? 512 : 256; }
 // doubles of a site's tables: ND orders x 6 points x 3 axes, made odd
 template <int MODE> struct GatherShape {
     static constexpr int ND = MODE == 0 ? 4 : 2;     // derivative orders needed
