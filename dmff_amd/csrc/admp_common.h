@@ -50,7 +50,8 @@ struct PcgState {
     double gam[2];  // r.z used by the update of that parity (+inf: restart the direction)
     double alp[2];  // step length of the update of that parity
     double res;     // max |r| over polarisable sites
-    int done, iter, pad0, pad1;
+    int done;       // not 0: converged (2 or 3: found by the update of parity 0 or 1)
+    int iter, pad0, pad1;
 };
 
 // Partial sums of the CG solve, per frame: nw slots of z.w, then r.z buffers 0

@@ -1057,19 +1057,18 @@ __global__ void __launch_bounds__(PCG_BLOCK) k_cg_update(int N, int nwu, int cur
                 }
             }
     }
-    // The flag of a frame that converged before.  Without PME no product tests the residual, and
-    // block 0 sets the flag below: the block takes what one of its threads read (at the barriers
-    // of the totals).
-    __shared__ int block_done;
-    if (threadIdx.x == 0) block_done = done;
+    // A frame that converged before.  Without PME no product tests the residual, and block 0
+    // sets the flag below, to a value of this parity: a wavefront that reads that value, from
+    // this launch or from one of this parity before, goes on like one that reads none and finds
+    // the residual of this parity below tol, as block 0 did (a converged frame's partials stay).
+    if (done && done != 2 + cur) return;
     double res, gamma, delta;
     parts_total_cg(parts.mx(f, cur), parts.rz(f, cur), parts.nb, parts.zw(f), nwu, sh, res, gamma, delta);
-    if (block_done) return;
     const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
     if (res < tol) {
         if (lead) {
             st[f].res = res;
-            st[f].done = 1;
+            st[f].done = 2 + cur;
         }
         return;
     }

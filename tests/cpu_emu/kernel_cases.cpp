@@ -21,46 +21,61 @@ template <class... KA, class... A> void one_block(void (*k)(KA...), dim3 g, dim3
     emu::end_kernel();
 }
 
-// the frame's flag, set by block 0 while another block of the launch runs
+// The frame's flag, set by block 0 (to the value that it leaves alone) while another block of the
+// launch runs, whose wavefronts then read it different.  run(block, residual) runs one block of an
+// update; a residual below tol (1) updates nothing, whenever the flag becomes visible.
 static PcgState g_st;
-static void set_done() { g_st.done = 1; }
-
-// k_jacobi, block 1 of 256: the residual is below tol, so nothing is updated, whenever block 0's
-// flag becomes visible.  (The launch before it leaves large maxima in LDS.)
-static int jacobi_flag() {
-    const int nb = 256, N = nb * 256;
-    std::vector<double> pol(N, 1.0), g(3 * N, 1.0), part(nb, 1e3), U(3 * N, 0.0);
+static int g_mark;
+template <class Run> static int flag_case(Run run, std::vector<double>& out) {
     int bad = 0;
-    for (int pass = 0; pass < 2; ++pass) {
-        g_st = PcgState{};
-        one_block(k_jacobi, dim3(nb), dim3(256), 1, N, 3, 1.0, pol.data(), g.data(), part.data(), U.data(), &g_st);
-        if (pass) for (double u : U) bad += u != 0.0;
-        std::fill(part.begin(), part.end(), 0.1);
-        std::fill(U.begin(), U.end(), 0.0);
-        emu::g_after_wave = set_done;
-    }
+    auto unchanged = [&] { for (double& v : out) { bad += v != 0.0; v = 0.0; } };
+    g_st = PcgState{};
+    run(0, 0.1);
+    g_mark = g_st.done;
+    bad += !g_mark;
+    unchanged();
+    g_st = PcgState{};
+    run(1, 1e3);            // leaves large values in LDS
+    std::fill(out.begin(), out.end(), 0.0);
+    g_st = PcgState{};
+    emu::g_after_wave = [] { g_st.done = g_mark; };
+    run(1, 0.1);
+    emu::g_after_wave = nullptr;
+    unchanged();
     return bad;
 }
 
-// k_cg_update, block 1 of 4, the same: the residual of parity 0 is below tol
+static int jacobi_flag() {
+    const int nb = 256, N = nb * 256;
+    std::vector<double> pol(N, 1.0), g(3 * N, 1.0), part(nb), U(3 * N, 0.0);
+    return flag_case([&](unsigned bx, double res) {
+        std::fill(part.begin(), part.end(), res);
+        one_block(k_jacobi, dim3(nb), dim3(256), bx, N, 3, 1.0, pol.data(), g.data(), part.data(), U.data(), &g_st);
+    }, U);
+}
+
 static int cg_flag() {
     const int nb = 4, N = nb * PCG_BLOCK, n3 = 3 * N;
     std::vector<double> pol(N, 1.0), x(n3, 0.0), r(2 * n3, 1e4), z(n3, 1.0), p(n3, 1.0), s(2 * n3, 1.0), w(n3, 1.0),
         rec(N * MREC, 0.0), parts(nb + 4 * nb, 1.0);
     const CgParts cp{parts.data(), nb, nb};
     BoxInfo box{};
-    std::fill(cp.mx(0, 0), cp.mx(0, 0) + nb, 1e3);
-    int bad = 0;
-    for (int pass = 0; pass < 2; ++pass) {
-        g_st = PcgState{};
-        one_block(k_cg_update<double>, dim3(nb), dim3(PCG_BLOCK), 1, N, nb, 0, 1.0, (const BoxInfo*)&box, pol.data(), x.data(),
-                  r.data(), z.data(), p.data(), s.data(), w.data(), rec.data(), (double*)nullptr, (const int*)nullptr,
-                  (const double*)nullptr, cp, &g_st);
-        if (pass) for (double v : x) bad += v != 0.0;
-        std::fill(cp.mx(0, 0), cp.mx(0, 0) + nb, 0.1);
-        std::fill(x.begin(), x.end(), 0.0);
-        emu::g_after_wave = set_done;
-    }
+    auto run = [&](int cur, unsigned bx) {
+        one_block(k_cg_update<double>, dim3(nb), dim3(PCG_BLOCK), bx, N, nb, cur, 1.0, (const BoxInfo*)&box, pol.data(),
+                  x.data(), r.data(), z.data(), p.data(), s.data(), w.data(), rec.data(), (double*)nullptr,
+                  (const int*)nullptr, (const double*)nullptr, cp, &g_st);
+    };
+    int bad = flag_case([&](unsigned bx, double res) {
+        std::fill(cp.mx(0, 0), cp.mx(0, 0) + nb, res);
+        run(0, bx);
+    }, x);
+    // the updates after it leave the frame alone, though parity 1 holds an older residual
+    std::fill(cp.mx(0, 1), cp.mx(0, 1) + nb, 1e3);
+    g_st = PcgState{};
+    run(0, 0);
+    for (int n = 1; n < 4; ++n)
+        for (unsigned bx = 0; bx < nb; ++bx) run(n & 1, bx);
+    for (double v : x) bad += v != 0.0;
     return bad;
 }
 
