@@ -483,8 +483,9 @@ static int spread_wpt(int K0, int K1, int K2, int F, int lm) {
 // 63 points (a third row tile), past the plane that fits the LDS (97^2), and past a z axis of 96
 // (the spread and the gather take a CU's LDS for one workgroup) they lose to radix passes whose
 // stages are short, i.e. axes of which no prime factor is above 5 (or 7 times a power of two);
-// with longer stages they win everywhere up to MM_KMAX (12,288 sites: 88 points 3.87 ms radix,
-// 2.05 here; 91: 5.15 and 2.32; 127: 785 and 13).  ms per evaluation, radix / here:
+// with longer stages they win, or are level but in batches past 100 points, up to MM_KMAX (one
+// frame of 12,288 sites: 88 points 3.24 ms radix, 2.05 here; 91: 3.86 and 2.31; 127: 147 and 4.0;
+// eight frames on 110 points: 17.8 and 20.3).  ms per evaluation, radix / here:
 //   solves, one frame of 12,288 sites: 80^3 2.32 / 2.03, 90^3 2.61 / 2.33, 80 x 80 x 120
 //     2.67 / 2.35, 96^3 2.88 / 3.02, 120^3 3.48 / 3.99, 128^3 4.33 / 5.68, 64 x 128 x 128
 //     3.01 / 3.30; of 98,304: 96^3 19.8 / 21.2, 128^3 24.5 / 27.1
