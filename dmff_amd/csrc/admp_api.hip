@@ -2354,12 +2354,17 @@ static PairParams make_pp(const double* mS, const double* pS, const double* dS, 
 }
 
 // The FP64 final pass without induced dipoles leaves registers to the reciprocal chain beside it:
-// for one frame, and for batches up to 32,768 sites, where the chain's launches are a large part
-// of the evaluation (12,288 sites, 50^3: 382 us with the register file full, 331 so; 98,304 sites
-// with 80 neighbours each, 80^3: 782 and 722; 8 frames of 3,000, 32^3: 379 and 352).  In larger
-// batches the pair pass itself counts for more (64 frames of 3,000: 1577 and 1630; 8 of 12,288:
-// 1259 and 1292).
-static bool real_final_room(const admp_ctx* ctx) { return ctx->F == 1 || (long)ctx->N * ctx->F <= 32768; }
+// for one frame, for batches up to 65,536 sites, and up to 131,072 sites on grids of more than 16
+// points per site, where the chain's launches are a large part of the evaluation (us, register
+// file full / room left: 12,288 sites, 50^3, 10 A: 382 / 331; 98,304 sites, 80^3, 6 A: 782 / 722;
+// 8 frames of 3,000, 32^3: 379 / 352; 4 of 12,288, 48^3: 602 / 545; 8 of 12,288, 64^3: 1028 / 935,
+// 100^3: 1578 / 1500).  Elsewhere the pair pass itself counts for as much or more (64 frames of
+// 3,000, 32^3: 1577 / 1630; 8 of 12,288, 50^3, 10 A: 1259 / 1292; 32 of 12,288, 48^3: 2973 / 3052,
+// 80^3: 4060 / 4147).
+static bool real_final_room(const admp_ctx* ctx) {
+    const long nf = (long)ctx->N * ctx->F;
+    return ctx->F == 1 || nf <= 65536 || (nf <= 131072 && ctx->eg.G > 16 * (size_t)ctx->N);
+}
 
 template <class R>
 static admp_status compute_impl(admp_ctx* ctx, const double* Q_local, const double* pol, const double* thole,

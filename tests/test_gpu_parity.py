@@ -615,9 +615,9 @@ def test_grids_beside_the_radix_line(K):
     assert errs.pop("E") < 1e-9 and max(errs.values()) < 1e-7
 
 
-@pytest.mark.parametrize("n_frames", [248, 249])
+@pytest.mark.parametrize("n_frames", [992, 993])
 def test_final_pass_of_batches_without_dipoles(n_frames):
-    """248 frames of 132 sites (32,736) leave registers to the reciprocal chain, 249 fill the register
+    """992 frames of 132 sites (130,944) leave registers to the reciprocal chain, 993 fill the register
     file: both are the single frames (same terms in the same order: 1e-13 relative)."""
     from dmff_amd.admp.engine import Engine
     s, pos, box = _small_waters()
